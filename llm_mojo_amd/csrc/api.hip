@@ -59,6 +59,7 @@ int ctx_workspace(llmq_ctx *ctx, size_t bytes, void **p, int slot) {
         ctx->ws_bytes[slot] = want;
     }
     *p = ctx->ws[slot];
+    ctx->ws_used = true;
     return LLMQ_OK;
 }
 
@@ -100,6 +101,7 @@ int llmq_destroy(llmq_ctx *ctx) {
     hipStreamSynchronize(ctx->stream);
     for (void *p : ctx->ws)
         if (p) hipFree(p);
+    if (ctx->ws_event) hipEventDestroy(ctx->ws_event);
     if (ctx->own_stream) hipStreamDestroy(ctx->own_stream);
     delete ctx;
     return LLMQ_OK;
@@ -107,7 +109,20 @@ int llmq_destroy(llmq_ctx *ctx) {
 
 int llmq_set_stream(llmq_ctx *ctx, void *s) {
     LLMQ_REQUIRE(ctx, "set_stream: null context");
-    ctx->stream = s ? (hipStream_t)s : ctx->own_stream;
+    const hipStream_t to = s ? (hipStream_t)s : ctx->own_stream;
+    if (to != ctx->stream && ctx->ws_used) {
+        // the workspaces are shared by every stream the context is given: work on the new one waits
+        // for what is still reading them on the old one (not within a capture, which cannot wait on it)
+        hipStreamCaptureStatus a = hipStreamCaptureStatusNone, b = a;
+        if (hipStreamIsCapturing(ctx->stream, &a) == hipSuccess && hipStreamIsCapturing(to, &b) == hipSuccess &&
+            a == hipStreamCaptureStatusNone && b == hipStreamCaptureStatusNone &&
+            (ctx->ws_event || hipEventCreateWithFlags(&ctx->ws_event, hipEventDisableTiming) == hipSuccess) &&
+            hipEventRecord(ctx->ws_event, ctx->stream) == hipSuccess)
+            (void)hipStreamWaitEvent(to, ctx->ws_event, 0);
+        (void)hipGetLastError();
+        ctx->ws_used = false;
+    }
+    ctx->stream = to;
     return LLMQ_OK;
 }
 

@@ -36,9 +36,11 @@ struct llmq_ctx {
     hipDeviceProp_t prop{};
     // grow-only workspaces: slot 0 the prompt-side int16 activation codes
     // (and LayerNorm outputs), slot 1 the fp16 activation records of the
-    // several-token Q4_K matmul
+    // several-token float-activation matmul
     void *ws[2] = {nullptr, nullptr};
     size_t ws_bytes[2] = {0, 0};
+    bool ws_used = false;           // handed out since the last change of stream
+    hipEvent_t ws_event = nullptr;  // llmq_set_stream orders the new stream after the workspaces' users
     void *scratch = nullptr;  // this device's no-allocation scratch (llmq_linear_noalloc), from llmq_init
 };
 
@@ -382,11 +384,14 @@ inline int float_act_type(const llmq_mat *w) {
 // log2 of the chunks per group of a QuantMatrix (31 for per-channel: every
 // chunk of a row is group 0); groups are powers of two times 32 otherwise.
 int qm_cpg_shift(const llmq_mat *w);
-// Several-token GGUF matmul on the fp32 matrix cores (gguf_gemm.hip).
-// Q4_K matrices with whole superblocks take the fp16 matrix cores over an
-// h16 record of x (gguf_gemm16.hip): `rec` of `rec_cap` bytes when given,
-// the context's workspace slot 1 when rec_cap < 0, and the fp32 kernel when
-// rec_cap == 0 (callers that may not allocate); LLMQ_GEMM_H16=0 forces the
+// Several-token GGUF matmul.  Matrices of whole superblocks take the fp16
+// matrix cores over an h16 record of x (gguf_gemm16.hip for a few tokens of
+// Q4_K, gemm_planes.hip): `rec` of `rec_cap` bytes when given, the context's
+// workspace slot 1 when rec_cap < 0, and the fp32 matrix cores
+// (gguf_gemm.hip) when rec_cap == 0; LLMQ_GEMM_H16=0 forces those.  Types
+// other than Q4_K need no record to be accepted: without room for one, and
+// under graph capture over the context's workspace (which a later call may
+// move), they take as many tokens at a time as there is room for, or the
 // fp32 kernel.
 int launch_gguf_gemm(llmq_ctx *ctx, const llmq_mat *w, const float *x, int64_t ldx, int64_t T, float *out,
                      int64_t ldo, const float *bias, int flags, void *rec = nullptr, int64_t rec_cap = -1);
@@ -395,7 +400,17 @@ int launch_gguf_gemm(llmq_ctx *ctx, const llmq_mat *w, const float *x, int64_t l
 int64_t h16_rec_bytes(int64_t T, int64_t K);
 void h16_rec_parts(void *rec, int64_t T, int64_t K, uint8_t **planes, _Float16 **sums, float **inv);
 bool gguf_gemm_h16_ok(const llmq_mat *w);
-int launch_act_h16(llmq_ctx *ctx, const float *x, int64_t ldx, int64_t T, int64_t K, void *rec);
+// The matmul over that record for prompts and the other float-activation
+// formats (gemm_planes.hip): any GGUF or A16 = False matrix of whole
+// superblocks whose groups are a power of two times 32 or the row.
+// gemm_planes_tile is the tile for T tokens, or -1 where the fp32 kernel is
+// the faster one; an output's bits depend on the tile and its own token only.
+bool gemm_planes_ok(const llmq_mat *w);
+int gemm_planes_tile(const llmq_mat *w, int64_t T);
+int launch_gemm_planes(llmq_ctx *ctx, const llmq_mat *w, const void *rec, int64_t T, float *out, int64_t ldo,
+                       const float *bias, int flags, int tile);
+// (rows: a wave a superblock of a token, for one token tile of Q4_K)
+int launch_act_h16(llmq_ctx *ctx, const float *x, int64_t ldx, int64_t T, int64_t K, void *rec, bool rows = false);
 // The batch-decode chain's forms of that matmul (gguf_gemm16.hip): the
 // input may be an "h16s" record (a scale per 16 inputs of a token, written
 // by the previous matmul's epilogue), its outputs then times each token's

@@ -1,0 +1,586 @@
+// Several-token matmul on the fp16 matrix cores over activation planes: the
+// kernel template behind gemm_planes_*.hip.
+//
+// One kernel covers every stored weight format whose codes, less their zero
+// point (and times an integer sub-block scale), are exact in fp16.  The
+// activations come as the h16 record of gguf_gemm16.hip: per token and
+// superblock of 256 inputs a power-of-two scale s and x s as two fp16
+// planes, hi and lo (22 bits together).  v_mfma_f32_16x16x32_f16 then forms
+// sum q (hi + lo) with every product exact in its fp32 sums, and what is
+// left of the format is applied in fp32: the block's scale per chunk of 32
+// inputs (Q8_0, Q4_0, Q4_1, groups of 32), per group of 64 or 128, or once
+// a superblock (the K quants, one scale a row), then 1 / s per superblock.
+// The additive minima (Q4_1, Q4_K, Q5_K) are one more product per
+// superblock, over the record's sums of each chunk.  For Q4_K that product is
+// on whole numbers (m_j) in fp16; Q4_1 and Q5_K take their codes less 8 or 16
+// and the rest of the offset, in fp32, on the fp32 matrix cores, which keeps
+// the two large sums from cancelling (Q5_K 476 x 768 x 2304: 4.8e-7 off the
+// 64-bit result without, the fp32 kernel before 2.9e-7).
+//
+// Mapping: a workgroup of WT x WR x WK waves owns WT TT token tiles and
+// WR RT row tiles (16 each); a wave computes TT x RT of the 16 x 16 blocks,
+// over the whole reduction axis (WK = 1) or every WK-th chunk of it (the
+// waves' sums are then added in LDS, in wave order), so an output's bits do
+// not depend on the other tokens of the call.  The axis is walked in steps
+// of S chunks: a step's planes, codes and scales are copied into one of two
+// LDS buffers (global-to-LDS loads) while the waves compute the other; a
+// superblock's fields, sums and 1 / s go to a pair of buffers of their own.
+//
+// What bounds it: per chunk, a wave reads 2 KB of planes a token tile and
+// decodes a row tile's codes (10-20 vector instructions) for 2 TT RT
+// products of 16 cycles each.  With RT = 4 the LDS reads take half of the
+// products' time; the decode and the scales (4 fma a block and chunk) come
+// to the products' own time at TT = 2 and stay below it at TT = 4, which
+// only the formats with one scale a superblock have registers for.  Small
+// calls are bound by one wave's chain through a chunk (read, decode, two
+// products, scale: ~0.15 us): more, smaller workgroups, and below ~250 of
+// them waves that share the chunks out (WK = 4).  Three or four buffers in
+// flight instead of two measured the same or slower at every size.
+// 512 x 4096 x 11008: Q8_0 1058 us on the fp32 matrix cores, 126 here
+// (0.73 PFLOP/s of fp16 products); Q6_K 1175 -> 160, Q5_K 777 -> 148,
+// Q4_0 1137 -> 115, Q4_1 1135 -> 135, int8-ch 1147 -> 114.
+#pragma once
+#include <type_traits>
+
+#include "common.h"
+
+namespace planes {
+
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+
+enum Fmt { kQ8_0, kQ4_0, kQ4_1, kQ4_K, kQ5_K, kQ6_K, kQm4, kQm8 };
+
+struct Args {
+    const uint8_t *planes, *sums, *inv;        // the h16 record
+    const uint8_t *codes, *scales, *zps, *bits, *sb, *sbd;
+    int T, n, ntiles, NC, NSB, NG, gshift, flags;  // NC chunks of 32 inputs, NSB superblocks, NG groups a row
+    int rows_first;                                // workgroup order: row blocks fastest
+    int64_t ldo;
+    const float *bias;
+    float *out;
+};
+
+// Bytes a format keeps per (16-row tile, chunk of 32 inputs) and superblock.
+template <int F>
+struct Tr {
+    static constexpr bool KQ = F == kQ4_K || F == kQ5_K || F == kQ6_K;
+    static constexpr bool QM = F == kQm4 || F == kQm8;
+    static constexpr bool W8 = F == kQ8_0 || F == kQm8;
+    static constexpr int CB = W8 ? 512 : 256;                               // codes
+    static constexpr int SCB = KQ ? 0 : F == kQ4_1 ? 64 : 32;               // scales
+    static constexpr int ZB = QM ? 16 : 0;                                  // zero points
+    static constexpr int HB = F == kQ5_K ? 64 : F == kQ6_K ? 128 : 0;       // high bits
+    static constexpr int SBF = KQ ? 256 : 0, SBD = F == kQ6_K ? 32 : 0;     // superblock fields
+    static constexpr bool SUMS = F == kQ4_1 || F == kQ4_K || F == kQ5_K;    // additive minima
+    static constexpr bool CENTER = F == kQ4_1 || F == kQ5_K;                // codes less 8 / 16, minima in fp32
+};
+
+// 1024 + the 8 bytes of (a, b) as fp16 pairs (a0, a1), (a2, a3), (b0, b1),
+// (b2, b3): 0x6400 | n is 1024 + n in fp16 for n < 1024.
+__device__ __forceinline__ void bytes_f16(uint32_t a, uint32_t b, v2h (&d)[4]) {
+    d[0] = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(0x64646464u, a, 0x04010400u));
+    d[1] = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(0x64646464u, a, 0x04030402u));
+    d[2] = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(0x64646464u, b, 0x04010400u));
+    d[3] = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(0x64646464u, b, 0x04030402u));
+}
+__device__ __forceinline__ float h2f(uint32_t bits) { return __half2float(__ushort_as_half((unsigned short)bits)); }
+// A read at byte `at` of an LDS buffer, the whole offset as one index: the
+// compiler keeps track of which buffer a read is from (and so does not make
+// it wait for copies into the others) through a few address steps only.
+template <class T>
+__device__ __forceinline__ T lds(const uint8_t *buf, int at) {
+    return *reinterpret_cast<const T *>(buf + at);
+}
+__device__ __forceinline__ v2h splat(float v) { return (v2h){(_Float16)v, (_Float16)v}; }
+
+template <int F, int TT, int RT, int WT, int WR, int S>
+struct Lay {
+    using R = Tr<F>;
+    static constexpr int NTT = WT * TT, NRT = WR * RT;
+    static constexpr int A = NTT * S * 2048, C = NRT * S * R::CB, SC = NRT * S * R::SCB, Z = NRT * S * R::ZB,
+                         H = NRT * S * R::HB;
+    static constexpr int oC = A, oSC = oC + C, oZ = oSC + SC, oH = oZ + Z, STEP = oH + H;
+    static constexpr int SBF = NRT * R::SBF, SBD = NRT * R::SBD, SU = R::SUMS ? NTT * 512 : 0, IV = NTT * 64;
+    static constexpr int oSBD = SBF, oSU = oSBD + SBD, oIV = oSU + SU, SBUF = oIV + IV;
+};
+
+// SEG: chunks of 32 inputs that share a scale (1, 2, 4, or 8 for one scale a
+// superblock or more).
+template <int F, int SEG0, int TT, int RT, int WT, int WR, int WK, int S>
+__global__ __launch_bounds__(WT * WR * WK * 64, 2) void gemm_planes_kernel(Args a) {
+    using R = Tr<F>;
+    using L = Lay<F, TT, RT, WT, WR, S>;
+    constexpr int SPB = 8 / S;  // steps a superblock
+    static_assert(8 % S == 0 && S % WK == 0 && 4 % WK == 0, "whole steps a superblock, chunks for every wave");
+    constexpr int NW = WT * WR * WK, RB = NW * 1024;  // bytes a copy round: 16 a lane
+    // (waves that share a group's chunks scale each by itself)
+    constexpr int SEG = WK > 1 && SEG0 < 8 ? 1 : SEG0;
+    constexpr bool CHAIN = R::KQ || SEG == 8;    // one scale a superblock: the products of all 8 chunks chain
+    // separate arrays, so that the compiler sees a copy into one cannot alias reads of another
+    __shared__ __align__(16) uint8_t b0[L::STEP], b1[L::STEP], f0[L::SBUF], f1[L::SBUF];
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int c16 = lane & 15, g = lane >> 4;
+    const int wt = w / WR % WT, wr = w % WR, kk = w / (WT * WR);
+    // Workgroups go to the 8 XCDs in turn (linear id mod 8); each XCD gets a
+    // contiguous run of (token block, row block) pairs, the operand with
+    // more bytes slowest, so that it is read by few XCDs.
+    int bx, by;
+    {
+        const int gx = gridDim.x, gy = gridDim.y, nb = gx * gy, id = blockIdx.y * gx + blockIdx.x;
+        const int x = id & 7, q = nb >> 3, rem = nb & 7, pos = x * q + min(x, rem) + (id >> 3);
+        if (a.rows_first) {
+            bx = pos % gx;
+            by = pos / gx;
+        } else {
+            by = pos % gy;
+            bx = pos / gy;
+        }
+    }
+    const int rt0 = bx * L::NRT, tt0 = by * L::NTT, ttiles = (a.T + 15) >> 4;
+    // A token tile past the record or a row tile past the matrix copies tile
+    // 0 instead (its outputs are not stored).
+    auto ttile = [&](int j) __attribute__((always_inline)) { return tt0 + j < ttiles ? tt0 + j : 0; };
+    auto rtile = [&](int j) __attribute__((always_inline)) { return rt0 + j < a.ntiles ? rt0 + j : 0; };
+    // One region's copy: the 16 bytes at region offset off(q) from voff[q] on
+    // from src; a last partial round is shared out over all waves where it
+    // divides.
+    auto part = [](int N, int q) constexpr { return q < N / RB || N % RB % (16 * NW) ? 1024 : N % RB / NW; };
+    auto off = [&](auto bytes, int q) __attribute__((always_inline)) {
+        return q * RB + w * part(decltype(bytes)::value, q) + lane * 16;
+    };
+    auto copy = [&](const uint8_t *src, uint8_t *dst, auto bytes, const uint32_t *voff) __attribute__((always_inline)) {
+        constexpr int N = decltype(bytes)::value;
+#pragma unroll
+        for (int q = 0; q < (N + RB - 1) / RB; q++) {
+            const bool whole = (q + 1) * RB <= N;
+            if (whole || (N % RB % (16 * NW) ? off(bytes, q) < N : lane * 16 < part(N, q)))
+                __builtin_amdgcn_global_load_lds(src + voff[q],
+                                                 (__attribute__((address_space(3))) void *)(dst + q * RB + w * part(N, q)), 16, 0, 0);
+        }
+    };
+    constexpr int NA = (L::A + RB - 1) / RB, NCC = (L::C + RB - 1) / RB, NS = (L::SC + RB - 1) / RB,
+                  NZ = (L::Z + RB - 1) / RB, NH = (L::H + RB - 1) / RB, NF = (L::SBF + RB - 1) / RB;
+#define LLMQ_N(bytes) std::integral_constant<int, bytes>{}
+    uint32_t vA[NA], vC[NCC], vS[NS ? NS : 1], vZ[NZ ? NZ : 1], vH[NH ? NH : 1], vF[NF ? NF : 1], vD[1], vU[1], vI[1];
+#pragma unroll
+    for (int q = 0; q < NA; q++) {
+        const int x = off(LLMQ_N(L::A), q);
+        vA[q] = ttile(x / (S * 2048)) * a.NC * 2048 + x % (S * 2048);
+    }
+#pragma unroll
+    for (int q = 0; q < NCC; q++) {
+        const int x = off(LLMQ_N(L::C), q);
+        vC[q] = rtile(x / (S * R::CB)) * a.NC * R::CB + x % (S * R::CB);
+    }
+    if constexpr (R::SCB > 0 && !R::QM) {
+#pragma unroll
+        for (int q = 0; q < NS; q++) {
+            const int x = off(LLMQ_N(L::SC), q);
+            vS[q] = rtile(x / (S * R::SCB)) * a.NC * R::SCB + x % (S * R::SCB);
+        }
+    }
+    if constexpr (R::HB > 0) {
+#pragma unroll
+        for (int q = 0; q < NH; q++) {
+            const int x = off(LLMQ_N(L::H), q);
+            vH[q] = rtile(x / (S * R::HB)) * a.NC * R::HB + x % (S * R::HB);
+        }
+    }
+    if constexpr (R::SBF > 0) {
+#pragma unroll
+        for (int q = 0; q < NF; q++) {
+            const int x = off(LLMQ_N(L::SBF), q);
+            vF[q] = rtile(x / 256) * a.NSB * 256 + x % 256;
+        }
+    }
+    static_assert(L::SBD <= RB && L::SU <= RB && L::IV <= RB, "one copy round each");
+    if constexpr (R::SBD > 0) {
+        const int x = off(LLMQ_N(L::SBD), 0);
+        vD[0] = rtile(x / 32) * a.NSB * 32 + x % 32;
+    }
+    if constexpr (R::SUMS) {
+        const int x = off(LLMQ_N(L::SU), 0);
+        vU[0] = ttile(x / 512) * a.NSB * 512 + x % 512;
+    }
+    {
+        const int x = off(LLMQ_N(L::IV), 0);
+        vI[0] = ttile(x / 64) * a.NSB * 64 + x % 64;
+    }
+#define LLMQ_CP(base, dst, bytes, v, at) copy(base + (int64_t)(at), dst, LLMQ_N(bytes), v)
+    auto stage = [&](int c0, uint8_t *buf) __attribute__((always_inline)) {  // chunks c0 .. c0 + S - 1
+        LLMQ_CP(a.planes, buf, L::A, vA, c0 * 2048);
+        LLMQ_CP(a.codes, buf + L::oC, L::C, vC, c0 * R::CB);
+        if constexpr (R::QM) {  // the chunk's group
+#pragma unroll
+            for (int q = 0; q < NS; q++) {
+                const int x = off(LLMQ_N(L::SC), q), u = x % (S * 32) / 32;
+                vS[q] = (rtile(x / (S * 32)) * a.NG + ((c0 + u) >> a.gshift)) * 32 + x % 32;
+            }
+#pragma unroll
+            for (int q = 0; q < NZ; q++) {
+                const int x = off(LLMQ_N(L::Z), q), u = x % (S * 16) / 16;
+                vZ[q] = (rtile(x / (S * 16)) * a.NG + ((c0 + u) >> a.gshift)) * 16;
+            }
+            LLMQ_CP(a.scales, buf + L::oSC, L::SC, vS, 0);
+            LLMQ_CP(a.zps, buf + L::oZ, L::Z, vZ, 0);
+        } else if constexpr (R::SCB > 0) {
+            LLMQ_CP(a.scales, buf + L::oSC, L::SC, vS, c0 * R::SCB);
+        }
+        if constexpr (R::HB > 0) LLMQ_CP(a.bits, buf + L::oH, L::H, vH, c0 * R::HB);
+    };
+    auto stage_sb = [&](int sb, uint8_t *buf) __attribute__((always_inline)) {
+        if constexpr (R::SBF > 0) LLMQ_CP(a.sb, buf, L::SBF, vF, sb * 256);
+        if constexpr (R::SBD > 0) LLMQ_CP(a.sbd, buf + L::oSBD, L::SBD, vD, sb * 32);
+        if constexpr (R::SUMS) LLMQ_CP(a.sums, buf + L::oSU, L::SU, vU, sb * 512);
+        LLMQ_CP(a.inv, buf + L::oIV, L::IV, vI, sb * 64);
+    };
+#undef LLMQ_CP
+    const v4f zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    v4f acc[TT][RT], d[TT][RT];  // outputs; the superblock's sums in scale s
+#pragma unroll
+    for (int t = 0; t < TT; t++)
+#pragma unroll
+        for (int r = 0; r < RT; r++) acc[t][r] = zero;
+    v4f seg[TT][RT];                // SEG 2, 4: the group's sums
+    v2h sc[RT][4];                  // K quants: sub-block scales (sc_2i, sc_2i+1); Q6_K: from LDS
+    uint32_t mp[RT][4];             // Q4_K: minima of the 8 chunks, fp16 pairs
+    float cm[RT][2] = {};           // CENTER: the offsets of chunks g and 4 + g
+    float rs[RT];                   // SEG 8: the row's scale
+
+    // this lane's place in each region of a buffer (opaque, so that a read is one step from its buffer)
+    auto place = [](int v) { asm("" : "+v"(v)); return v; };
+    const int pA = place(wt * TT * S * 2048 + kk * 2048 + lane * 16);
+    const int pC = place(L::oC + wr * RT * S * R::CB + kk * R::CB + (R::W8 ? (g >> 1) * 256 + c16 * 16 + (g & 1) * 8 : c16 * 16 + g * 4));
+    const int pS = place(L::oSC + wr * RT * S * R::SCB + kk * R::SCB + c16 * (R::SCB / 16));
+    const int pZ = place(L::oZ + wr * RT * S * 16 + kk * 16 + c16);
+    const int pH = place(L::oH + wr * RT * S * R::HB + kk * R::HB + c16 * (R::HB / 16) + g * (R::HB / 64));
+    const int pF = place(wr * RT * 256 + c16 * 16), pF6 = place(wr * RT * 256 + c16 * 16 + (g >> 1) + 2 * kk);
+    const int pD = place(L::oSBD + wr * RT * 32 + c16 * 2);
+    const int pU = place(L::oSU + wt * TT * 512 + (R::CENTER ? c16 * 16 + g * 2 : (lane & 31) * 16));
+    const int pI = place(L::oIV + wt * TT * 64 + g * 16);
+
+    // row tile r's sums x of chunk j (or of its group, at the last) times the scale s
+    auto scale = [&](int j, int r, const v4f (&x)[TT], float s) __attribute__((always_inline)) {
+#pragma unroll
+        for (int t = 0; t < TT; t++) {
+            if (SEG == 1 || (j + 1) % SEG == 0) {
+#pragma unroll
+                for (int i = 0; i < 4; i++) d[t][r][i] = j < SEG ? s * x[t][i] : fmaf(s, x[t][i], d[t][r][i]);
+                asm volatile("" : "+v"(d[t][r]));  // (formed here: sunk past a branch, its products' results would pile up)
+            } else {
+                seg[t][r] = x[t];
+            }
+        }
+    };
+
+    // chunks j0 .. j0 + S - 1 of a superblock from cur, its fields in sbf
+    auto compute = [&](auto j0c, const uint8_t *cur, const uint8_t *sbf) __attribute__((always_inline)) {
+        constexpr int j0 = decltype(j0c)::value;
+        if constexpr ((F == kQ4_K || F == kQ5_K) && j0 == 0) {
+#pragma unroll
+            for (int r = 0; r < RT; r++) {
+                // sc_j and m_j as bytes (k_scale_min, gguf.mojo:205-221, four at a time)
+                const uint4 f = lds<uint4>(sbf, pF + r * 256);
+                const uint32_t sl = f.y & 0x3F3F3F3Fu, ml = f.z & 0x3F3F3F3Fu;
+                const uint32_t sh = (f.w & 0x0F0F0F0Fu) | ((f.y >> 2) & 0x30303030u);
+                const uint32_t mh = ((f.w >> 4) & 0x0F0F0F0Fu) | ((f.z >> 2) & 0x30303030u);
+                if constexpr (WK > 1)  // this wave's chunks' bytes to each unit's first place
+                    bytes_f16(sl >> (8 * kk), sh >> (8 * kk), sc[r]);
+                else
+                    bytes_f16(sl, sh, sc[r]);
+#pragma unroll
+                for (int i = 0; i < 4; i++) sc[r][i] = sc[r][i] - splat(1024.0f);
+                if constexpr (F == kQ4_K) {
+                    v2h m2[4];
+                    bytes_f16(ml, mh, m2);
+#pragma unroll
+                    for (int i = 0; i < 4; i++) mp[r][i] = __builtin_bit_cast(uint32_t, m2[i] - splat(1024.0f));
+                } else if (kk == 0) {  // 16 d sc - dmin m of chunks g and 4 + g
+                    const float d16 = 16.0f * h2f(f.x & 0xFFFFu), dmin = h2f(f.x >> 16);
+                    cm[r][0] = fmaf(d16, (float)((sl >> (8 * g)) & 255u), -dmin * (float)((ml >> (8 * g)) & 255u));
+                    cm[r][1] = fmaf(d16, (float)((sh >> (8 * g)) & 255u), -dmin * (float)((mh >> (8 * g)) & 255u));
+                }
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < S; u += WK) {
+            const int j = j0 + u;  // this wave's chunk is j + kk
+            v4f px[TT];
+            float ps = 0.0f;
+            uint4 ah[TT], al[TT];
+#pragma unroll
+            for (int t = 0; t < TT; t++) {
+                const int p = pA + (t * S + u) * 2048;
+                ah[t] = lds<uint4>(cur, p);
+                al[t] = lds<uint4>(cur, p + 1024);
+            }
+#pragma unroll
+            for (int r = 0; r < RT; r++) {
+                const int e = r * S + u;  // (row tile, chunk) entry
+                // the 8 codes of row c16, inputs 8 g .. 8 g + 7, as 1024 + code in fp16, inputs 0 2 4 6 1 3 5 7
+                uint32_t ev, od;
+                if constexpr (R::W8) {
+                    const uint2 cw = lds<uint2>(cur, pC + e * 512);
+                    ev = __builtin_amdgcn_perm(cw.y, cw.x, 0x06040200u);
+                    od = __builtin_amdgcn_perm(cw.y, cw.x, 0x07050301u);
+                    if constexpr (F == kQ8_0) {  // int8 + 128
+                        ev ^= 0x80808080u;
+                        od ^= 0x80808080u;
+                    }
+                } else {
+                    const uint32_t cw = lds<uint32_t>(cur, pC + e * 256);
+                    ev = cw & 0x0F0F0F0Fu;
+                    od = (cw >> 4) & 0x0F0F0F0Fu;
+                }
+                if constexpr (F == kQ5_K) {
+                    // bits 0, 2, 4, 6 of the group's byte to bit 4 of four bytes (the product's other terms miss those)
+                    const uint32_t hb = lds<uint8_t>(cur, pH + e * 64);
+                    ev |= __umul24(hb & 0x55u, 0x00410410u) & 0x10101010u;
+                    od |= __umul24((hb >> 1) & 0x55u, 0x00410410u) & 0x10101010u;
+                }
+                if constexpr (F == kQ6_K) {
+                    // two bits a code: bytes 0 and 1 of the group's halfword apart, then to bits 4, 5 of each code's byte
+                    const uint32_t h = lds<uint16_t>(cur, pH + e * 128);
+                    const uint32_t y = (h | (h << 8)) & 0x00FF00FFu;
+                    ev |= ((y << 4) & 0x00300030u) | ((y << 8) & 0x30003000u);
+                    od |= ((y << 2) & 0x00300030u) | ((y << 6) & 0x30003000u);
+                }
+                v2h q[4];
+                bytes_f16(ev, od, q);
+                v8h b, be;  // the weights; Q6_K: what fp16 leaves of sc q beyond 2048
+                if constexpr (F == kQ4_K) {
+                    // (1024 + u) sc - 1024 sc = u sc exactly (below 2048)
+                    const _Float16 s1 = sc[r][j >> 1][j & 1], n1 = s1 * (_Float16)-1024.0f;
+                    const v2h sv = {s1, s1}, nv = {n1, n1};
+#pragma unroll
+                    for (int i = 0; i < 4; i++) q[i] = __builtin_elementwise_fma(q[i], sv, nv);
+                } else if constexpr (F == kQ5_K) {
+                    const _Float16 s1 = sc[r][j >> 1][j & 1];
+                    const v2h sv = {s1, s1};
+#pragma unroll
+                    for (int i = 0; i < 4; i++) q[i] = (q[i] - splat(1040.0f)) * sv;  // (u - 16) sc, below 1024
+                } else if constexpr (F == kQ6_K) {
+                    // sub-block 2 j + g / 2's int8 scale; |sc q| <= 4096: rounded to fp16 and the rest (-1, 0, 1)
+                    const _Float16 s1 = (_Float16)(short)lds<int8_t>(sbf, pF6 + r * 256 + 2 * j);
+                    const v2h sv = {s1, s1};
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        const v2h c = q[i] - splat(1056.0f);
+                        q[i] = c * sv;
+                        const v2h x = __builtin_elementwise_fma(c, sv, -q[i]);
+                        be[2 * i] = x[0];
+                        be[2 * i + 1] = x[1];
+                    }
+                } else {
+                    v2h z = splat(F == kQ8_0 ? 1152.0f : F == kQ4_0 || F == kQ4_1 ? 1032.0f : 1024.0f);
+                    if constexpr (R::QM)
+                        z = __builtin_bit_cast(v2h, (uint32_t)lds<uint8_t>(cur, pZ + e * 16) * 0x10001u + 0x64006400u);
+#pragma unroll
+                    for (int i = 0; i < 4; i++) q[i] = q[i] - z;
+                }
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    b[2 * i] = q[i][0];
+                    b[2 * i + 1] = q[i][1];
+                }
+                float s = 0.0f;
+                if constexpr (F == kQ4_1) {
+                    const uint32_t m = lds<uint32_t>(cur, pS + e * 64);
+                    s = h2f(m & 0xFFFFu);
+                    const float c = fmaf(8.0f, s, h2f(m >> 16));  // lane group j % 4 keeps chunk j's
+                    cm[r][j >> 2] = (j & 3) + kk == g ? c : cm[r][j >> 2];
+                } else if constexpr (!R::KQ) {
+                    if ((j + WK) % SEG == 0) s = h2f(lds<uint16_t>(cur, pS + e * 32));
+                    if (SEG == 8 && j + WK == 8) rs[r] = s;
+                }
+                v4f x[TT];
+#pragma unroll
+                for (int t = 0; t < TT; t++) {
+                    const v4f c = CHAIN ? (j == 0 ? zero : d[t][r]) : (j % SEG == 0 ? zero : seg[t][r]);
+                    x[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, ah[t]), b, c, 0, 0, 0);
+                }
+#pragma unroll
+                for (int t = 0; t < TT; t++)
+                    x[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, al[t]), b, x[t], 0, 0, 0);
+                if constexpr (F == kQ6_K) {
+#pragma unroll
+                    for (int t = 0; t < TT; t++)
+                        x[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, ah[t]), be, x[t], 0, 0, 0);
+                }
+                if constexpr (CHAIN) {
+#pragma unroll
+                    for (int t = 0; t < TT; t++) d[t][r] = x[t];
+                } else {
+                    // the scale of the block before this one (its products are done by now), and no
+                    // product ahead of it: more results in flight would not fit the registers
+                    if (r > 0) scale(j, r - 1, px, ps);
+#pragma unroll
+                    for (int t = 0; t < TT; t++) px[t] = x[t];
+                    ps = s;
+                    __builtin_amdgcn_sched_barrier(0x104);  // (LDS reads and scalar work may cross)
+                    if (r + 1 == RT) scale(j, r, px, ps);
+                }
+            }
+        }
+        if constexpr (j0 + S == 8) {  // the superblock's minima, scale and 1 / s
+            float dd[RT], dmin[RT];
+            v8h bm[RT];
+#pragma unroll
+            for (int r = 0; r < RT; r++) {
+                if constexpr (F == kQ5_K) {
+                    dd[r] = h2f(lds<uint16_t>(sbf, pF + r * 256));
+                } else if constexpr (F == kQ4_K) {
+                    const uint32_t f = lds<uint32_t>(sbf, pF + r * 256);
+                    dd[r] = h2f(f & 0xFFFFu);
+                    dmin[r] = -h2f(f >> 16);
+                } else if constexpr (F == kQ6_K) {
+                    dd[r] = h2f(lds<uint16_t>(sbf, pD + r * 32));
+                }
+                if constexpr (F == kQ4_K) {  // the minima in groups 0 and 1, against the sums' hi and lo planes
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        const v2h m2 = __builtin_bit_cast(v2h, g < 2 && kk == 0 ? mp[r][i] : 0u);
+                        bm[r][2 * i] = m2[0];
+                        bm[r][2 * i + 1] = m2[1];
+                    }
+                }
+            }
+#pragma unroll
+            for (int t = 0; t < TT; t++) {
+                const v4f iv = lds<v4f>(sbf, pI + t * 64);
+                uint4 sq = make_uint4(0u, 0u, 0u, 0u);
+                float xs[2] = {0.0f, 0.0f};
+                if constexpr (R::CENTER) {  // token c16's sums of chunks g and 4 + g
+                    const int p = pU + t * 512;
+                    xs[0] = (float)lds<_Float16>(sbf, p) + (float)lds<_Float16>(sbf, p + 256);
+                    xs[1] = (float)lds<_Float16>(sbf, p + 8) + (float)lds<_Float16>(sbf, p + 264);
+                } else if constexpr (R::SUMS) {
+                    sq = lds<uint4>(sbf, pU + t * 512);
+                    if (g >= 2) sq = make_uint4(0u, 0u, 0u, 0u);
+                }
+#pragma unroll
+                for (int r = 0; r < RT; r++) {
+                    v4f dm = zero;
+                    if constexpr (R::CENTER) {
+                        dm = __builtin_amdgcn_mfma_f32_16x16x4f32(xs[0], cm[r][0], zero, 0, 0, 0);
+                        dm = __builtin_amdgcn_mfma_f32_16x16x4f32(xs[1], cm[r][1], dm, 0, 0, 0);
+                    } else if constexpr (R::SUMS)
+                        dm = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, sq), bm[r], zero, 0, 0, 0);
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        float v = d[t][r][i];
+                        if constexpr (F == kQ4_K)
+                            v = fmaf(dmin[r], dm[i], dd[r] * v);
+                        else if constexpr (F == kQ5_K)
+                            v = fmaf(dd[r], v, dm[i]);
+                        else if constexpr (F == kQ6_K)
+                            v = dd[r] * v;
+                        else if constexpr (F == kQ4_1)
+                            v += dm[i];
+                        else if constexpr (SEG == 8)
+                            v = rs[r] * v;
+                        acc[t][r][i] = fmaf(iv[i], v, acc[t][r][i]);
+                    }
+                }
+            }
+        }
+    };
+    // One step: wait for its copies, start those of the next step into the
+    // buffer that the step before has left, compute.
+    auto step = [&](int sb, auto odd, auto j0c) __attribute__((always_inline)) {
+        constexpr int j0 = decltype(j0c)::value, P = decltype(odd)::value;
+        constexpr bool even = (P * SPB + j0 / S) % 2 == 0;
+        __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0), lgkmcnt(0): this wave's copies are in, its reads done
+        llmq_lds_barrier();
+        if (sb * 8 + j0 + S < a.NC) {
+            stage(sb * 8 + j0 + S, even ? b1 : b0);
+            if constexpr (j0 + S == 8) stage_sb(sb + 1, P ? f0 : f1);
+        }
+        compute(j0c, even ? b0 : b1, P ? f1 : f0);
+    };
+    auto superblock = [&](int sb, auto odd) __attribute__((always_inline)) {
+        step(sb, odd, LLMQ_N(0));
+        if constexpr (S == 2) step(sb, odd, LLMQ_N(2));
+        if constexpr (S <= 4) step(sb, odd, LLMQ_N(4));
+        if constexpr (S == 2) step(sb, odd, LLMQ_N(6));
+    };
+    stage(0, b0);
+    stage_sb(0, f0);
+    for (int sb = 0; sb < a.NSB; sb += 2) {
+        superblock(sb, LLMQ_N(0));
+        if (sb + 1 < a.NSB) superblock(sb + 1, LLMQ_N(1));
+    }
+#undef LLMQ_N
+    if constexpr (WK > 1) {  // the waves' sums over their chunks, in wave order
+        static_assert((WK - 1) * WT * WR * TT * RT * 1024 <= L::STEP, "the sums fit a step's buffer");
+        __syncthreads();
+        v4f *const p = reinterpret_cast<v4f *>(b0) + (w % (WT * WR)) * TT * RT * 64 + lane;
+        constexpr int KS = WT * WR * TT * RT * 64;
+        if (kk > 0) {
+#pragma unroll
+            for (int t = 0; t < TT; t++)
+#pragma unroll
+                for (int r = 0; r < RT; r++) p[(kk - 1) * KS + (t * RT + r) * 64] = acc[t][r];
+        }
+        __syncthreads();
+        if (kk > 0) return;
+#pragma unroll
+        for (int t = 0; t < TT; t++)
+#pragma unroll
+            for (int r = 0; r < RT; r++)
+#pragma unroll
+                for (int q = 0; q < WK - 1; q++) acc[t][r] += p[q * KS + (t * RT + r) * 64];
+    }
+    // store_out: bias, GELU, residual
+#pragma unroll
+    for (int r = 0; r < RT; r++) {
+        const int o = (rt0 + wr * RT + r) * 16 + c16;
+        const bool rok = o < a.n && rt0 + wr * RT + r < a.ntiles;
+        const float bo = rok && (a.flags & LLMQ_BIAS) ? a.bias[o] : 0.0f;
+#pragma unroll
+        for (int t = 0; t < TT; t++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int tok = (tt0 + wt * TT + t) * 16 + 4 * g + i;
+                if (!rok || tok >= a.T) continue;
+                float v = acc[t][r][i];
+                if (a.flags & LLMQ_BIAS) v += bo;
+                if (a.flags & LLMQ_GELU) v = gelu_ref(v);
+                float *dst = a.out + (int64_t)tok * a.ldo + o;
+                if (a.flags & LLMQ_RESID) v += *dst;
+                *dst = v;
+            }
+    }
+}
+
+// The tiles, as TT, RT, WT, WR, WK, S (kTiles in gemm_planes.hip has
+// what each costs).
+template <int F, int SEG>
+int launch_tile(hipStream_t st, int tile, const Args &a) {
+    const int tt = (a.T + 15) / 16, rt = a.ntiles;
+#define LLMQ_PK(TT, RT, WT, WR, WK, S)                                                                              \
+    hipLaunchKernelGGL((gemm_planes_kernel<F, SEG, TT, RT, WT, WR, WK, S>),                                     \
+                       dim3((unsigned)((rt + WR * RT - 1) / (WR * RT)), (unsigned)((tt + WT * TT - 1) / (WT * TT))), \
+                       dim3(WT *WR * WK * 64), 0, st, a)
+    switch (tile) {
+    case 0:  // (only where the registers hold it: one scale a superblock)
+        if constexpr (SEG == 8)
+            LLMQ_PK(4, 4, 1, 4, 1, 2);
+        else
+            LLMQ_PK(2, 4, 2, 2, 1, 2);
+        break;
+    case 1: LLMQ_PK(2, 4, 2, 2, 1, 2); break;
+    case 2: LLMQ_PK(2, 2, 2, 2, 1, 2); break;
+    case 3: LLMQ_PK(2, 1, 1, 4, 1, 4); break;
+    case 4: LLMQ_PK(1, 1, 1, 4, 1, 4); break;
+    case 5: LLMQ_PK(1, 1, 1, 4, 4, 8); break;
+    default: LLMQ_PK(1, 1, 1, 2, 4, 8); break;
+    }
+#undef LLMQ_PK
+    LLMQ_HIP(hipGetLastError());
+    return LLMQ_OK;
+}
+
+}  // namespace planes

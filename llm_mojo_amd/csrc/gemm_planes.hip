@@ -1,0 +1,148 @@
+// The activation-plane matmul (gemm_planes.h): which matrices it takes, the
+// tile of a call, and the operands.  The kernels are in gemm_planes_*.hip.
+#include "gemm_planes.h"
+
+namespace planes {
+
+#define LLMQ_PX(F, SEG) extern template int launch_tile<F, SEG>(hipStream_t, int, const Args &);
+LLMQ_PX(kQ8_0, 1) LLMQ_PX(kQ4_0, 1) LLMQ_PX(kQ4_1, 1) LLMQ_PX(kQ4_K, 8) LLMQ_PX(kQ5_K, 8) LLMQ_PX(kQ6_K, 8)
+LLMQ_PX(kQm4, 1) LLMQ_PX(kQm4, 2) LLMQ_PX(kQm4, 4) LLMQ_PX(kQm4, 8)
+LLMQ_PX(kQm8, 1) LLMQ_PX(kQm8, 2) LLMQ_PX(kQm8, 4) LLMQ_PX(kQm8, 8)
+#undef LLMQ_PX
+
+namespace {
+
+// Chunks of 32 inputs that share one of a QuantMatrix's scales, as the
+// kernel's SEG (8: one scale a superblock or more) and the shift from a
+// chunk to its group; false for groups the kernel does not take.
+bool qm_groups(const llmq_mat *w, int *seg, int *shift) {
+    if (w->NG == 1) {
+        *seg = 8;
+        *shift = 31;
+        return true;
+    }
+    const int64_t cpg = w->group / 32;
+    if (cpg < 1 || (cpg & (cpg - 1))) return false;
+    *shift = __builtin_ctzll((unsigned long long)cpg);
+    *seg = cpg < 8 ? (int)cpg : 8;
+    return true;
+}
+
+// A tile's size in 16-token and 16-row tiles, and what it measured on Q8_0
+// at 4096 x 4096 and 4096 x 11008: the time of a superblock in microseconds
+// with few workgroups, and how many of them run before that time grows.
+// (tile 0 on the K quants.)
+struct Tile {
+    int tt, rt;
+    float us, full;
+};
+constexpr Tile kTiles[] = {{4, 16, 5.2f, 280.0f}, {4, 8, 3.6f, 328.0f}, {4, 4, 2.4f, 386.0f}, {2, 4, 1.5f, 440.0f},
+                           {1, 4, 1.2f, 510.0f},  {1, 4, 0.7f, 275.0f}, {1, 2, 0.6f, 292.0f}};
+
+}  // namespace
+}  // namespace planes
+
+bool gemm_planes_ok(const llmq_mat *w) {
+    if (!w || !is_float_act(w) || w->k % 256 != 0) return false;
+    int seg, shift;
+    return w->kind == MAT_GGUF || planes::qm_groups(w, &seg, &shift);
+}
+
+// The tile with the least time by kTiles' figures; -1 where the fp32 kernel
+// is faster: it reads x itself, without the record's 4.5 us, at 22 MAC a
+// picosecond (16 tokens of 4096 x 4096: 12.3 us against 14, 64 tokens 50 against 18).
+// Q4_K has a kernel of its own for few tokens.
+int gemm_planes_tile(const llmq_mat *w, int64_t T) {
+    using namespace planes;
+    if (const char *e = getenv("LLMQ_PLANES_TILE")) {
+        const int t = atoi(e);
+        return t < 0 ? 0 : t > 6 ? 6 : t;
+    }
+    const int64_t tt = (T + 15) / 16;
+    int seg = 8, shift;
+    if (w->kind == MAT_QUANT) qm_groups(w, &seg, &shift);
+    const int ty = float_act_type(w);
+    const bool chain = seg == 8 && ty != LLMQ_GGML_Q8_0 && ty != LLMQ_GGML_Q4_0 && ty != LLMQ_GGML_Q4_1;
+    int best = -1;
+    float least = 0.0f;
+    for (int i = chain ? 0 : 1; i < (int)(sizeof(kTiles) / sizeof(kTiles[0])); i++) {
+        const Tile &k = kTiles[i];
+        const float wgs = (float)((tt + k.tt - 1) / k.tt * ((w->ntiles + k.rt - 1) / k.rt));
+        const float us = 4.5f + (float)(w->k / 256) * k.us * (wgs > k.full ? wgs / k.full : 1.0f);
+        if (best < 0 || us < least) {
+            best = i;
+            least = us;
+        }
+    }
+    const float fp32_us = 3.5f + (float)T * (float)w->k * (float)w->n / 22e6f;
+    return ty != LLMQ_GGML_Q4_K && fp32_us < least ? -1 : best;
+}
+
+int launch_gemm_planes(llmq_ctx *ctx, const llmq_mat *w, const void *rec, int64_t T, float *out, int64_t ldo,
+                       const float *bias, int flags, int tile) {
+    using namespace planes;
+    LLMQ_REQUIRE(gemm_planes_ok(w) && tile >= 0, "gemm_planes: not a matrix of this kernel");
+    LLMQ_REQUIRE(rec && out && T > 0, "gemm_planes: bad arguments");
+    LLMQ_REQUIRE(!(flags & LLMQ_BIAS) || bias, "gemm_planes: LLMQ_BIAS without a bias");
+    const int64_t T16 = (T + 15) / 16 * 16, NSB = w->k / 256;
+    const int64_t ntc = (w->ntiles * w->CK + LLMQ_PAD_CHUNKS) * 16, nts = (w->ntiles * w->NG + LLMQ_PAD_CHUNKS) * 16;
+    LLMQ_REQUIRE(ntc * 16 < (int64_t)kLlmqOOB && h16_rec_bytes(T, w->k) < (int64_t)kLlmqOOB,
+                 "gemm_planes: operands too large");
+    Args a{};
+    uint8_t *pl;
+    _Float16 *su;
+    float *iv;
+    h16_rec_parts(const_cast<void *>(rec), T, w->k, &pl, &su, &iv);
+    a.planes = pl;
+    a.sums = reinterpret_cast<const uint8_t *>(su);
+    a.inv = reinterpret_cast<const uint8_t *>(iv);
+    a.codes = w->codes;
+    int seg = 8;
+    if (w->kind == MAT_QUANT) {
+        qm_groups(w, &seg, &a.gshift);
+        a.scales = reinterpret_cast<const uint8_t *>(w->scales);
+        a.zps = w->zps;
+        a.NG = (int)w->NG;
+    } else if (w->ggml_type == LLMQ_GGML_Q4_1) {
+        a.scales = reinterpret_cast<const uint8_t *>(w->g_meta32);
+    } else if (w->ggml_type == LLMQ_GGML_Q8_0 || w->ggml_type == LLMQ_GGML_Q4_0) {
+        a.scales = reinterpret_cast<const uint8_t *>(w->g_meta16);
+    } else {
+        a.sb = reinterpret_cast<const uint8_t *>(w->g_sb16);
+        if (w->ggml_type == LLMQ_GGML_Q5_K) {
+            a.bits = reinterpret_cast<const uint8_t *>(w->g_bits32);
+        } else if (w->ggml_type == LLMQ_GGML_Q6_K) {
+            a.bits = reinterpret_cast<const uint8_t *>(w->g_bits64);
+            a.sbd = reinterpret_cast<const uint8_t *>(w->g_meta16);
+        }
+    }
+    a.T = (int)T;
+    a.n = (int)w->n;
+    a.ntiles = (int)w->ntiles;
+    a.NC = (int)(w->k / 32);
+    a.NSB = (int)NSB;
+    a.flags = flags;
+    a.rows_first = T16 * w->k * 4 > ntc * 16;
+    a.ldo = ldo;
+    a.bias = bias ? bias : out;
+    a.out = out;
+    hipStream_t st = ctx->stream;
+    switch (float_act_type(w)) {
+#define LLMQ_PS(F)                                             \
+    switch (seg) {                                             \
+    case 1: return launch_tile<F, 1>(st, tile, a);             \
+    case 2: return launch_tile<F, 2>(st, tile, a);             \
+    case 4: return launch_tile<F, 4>(st, tile, a);             \
+    default: return launch_tile<F, 8>(st, tile, a);            \
+    }
+    case kQmFloat4: LLMQ_PS(kQm4)
+    case kQmFloat8: LLMQ_PS(kQm8)
+#undef LLMQ_PS
+    case LLMQ_GGML_Q8_0: return launch_tile<kQ8_0, 1>(st, tile, a);
+    case LLMQ_GGML_Q4_0: return launch_tile<kQ4_0, 1>(st, tile, a);
+    case LLMQ_GGML_Q4_1: return launch_tile<kQ4_1, 1>(st, tile, a);
+    case LLMQ_GGML_Q4_K: return launch_tile<kQ4_K, 8>(st, tile, a);
+    case LLMQ_GGML_Q5_K: return launch_tile<kQ5_K, 8>(st, tile, a);
+    default: return launch_tile<kQ6_K, 8>(st, tile, a);
+    }
+}

@@ -1,0 +1,11 @@
+// The activation-plane matmul (gemm_planes.h) of int4 QuantMatrix with float activations.
+#include "gemm_planes.h"
+
+namespace planes {
+
+template int launch_tile<kQm4, 1>(hipStream_t, int, const Args &);
+template int launch_tile<kQm4, 2>(hipStream_t, int, const Args &);
+template int launch_tile<kQm4, 4>(hipStream_t, int, const Args &);
+template int launch_tile<kQm4, 8>(hipStream_t, int, const Args &);
+
+}  // namespace planes

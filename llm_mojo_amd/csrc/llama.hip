@@ -808,7 +808,7 @@ int ensure_rows(llmq_llama *m, int rows) {
     if (hipMalloc(&m->x, r * c.dim * 4) != hipSuccess || hipMalloc(&m->xn, r * c.dim * 4) != hipSuccess ||
         hipMalloc(&m->qkv, r * qkv_cols(c) * 4) != hipSuccess || hipMalloc(&m->att, r * c.dim * 4) != hipSuccess ||
         hipMalloc(&m->gu, r * 2 * c.ffn * 4) != hipSuccess || hipMalloc(&m->hh, r * c.ffn * 4) != hipSuccess ||
-        hipMalloc(&m->tokens, r * 8) != hipSuccess)
+        hipMalloc(&m->tokens, (r + 1) * 8) != hipSuccess)
         return llmq_set_error(LLMQ_ENOMEM, "llama: activations for %d tokens", rows);
     if (rows > 1) {
         const int64_t cap = h16_rec_bytes(rows, std::max(c.dim, c.ffn));
@@ -862,25 +862,28 @@ int norm_linear(llmq_llama *m, const float *g, const llmq_mat *w, int R, float *
 }
 
 // The layers for R = nseq * T rows in m->x: T tokens of sequences seq0 ..
-// at positions pos0 + t (prefill: nseq = 1), or one token of every
-// sequence at position state[0] (decode: T = 1, state given).
+// at positions pos0 + t (prefill: nseq = 1), or one token of R sequences
+// from seq0 at position state[0] (decode: T = 1, state given).
 // Decode attention of layer l for R sequences (RoPE, the cache store and
 // the attention over splits of kSplit positions in one launch); returns the
 // split count.
-int attend_splits(llmq_llama *m, int R, int l, const int *state) {
+int attend_splits(llmq_llama *m, int R, int l, const int *state, int seq0) {
     const llmq_llama_cfg &c = m->cfg;
     const int NS = (c.max_t + kSplit - 1) / kSplit, QC = qkv_cols(c);
     // LLMQ_ATTN_GROUP=1 / 0 forces the grouped / per-head kernel
     static const char *ge = getenv("LLMQ_ATTN_GROUP");
+    const int64_t at = (int64_t)seq0 * c.n_layer * c.n_kv * c.max_t;  // seq0's first cached row
+    int8_t *k8 = m->k8 + at * HD, *v8 = m->v8 + at * HD;
+    float *ks = m->ks + at, *vs = m->vs + at;
     const bool grouped = c.n_head == 8 * c.n_kv && (ge ? ge[0] == '1' : R > 1);
     if (grouped)  // the 8 query heads of a key / value head in one workgroup
         hipLaunchKernelGGL(attend_split_group_kernel, dim3(c.n_kv, R, NS), dim3(kSplit), 0, m->ctx->stream, m->qkv,
-                           (int64_t)QC, state, c.n_head, c.n_kv, c.n_layer, l, c.max_t, m->rope, m->k8, m->v8, m->ks,
-                           m->vs, m->apart, NS);
+                           (int64_t)QC, state, c.n_head, c.n_kv, c.n_layer, l, c.max_t, m->rope, k8, v8, ks, vs, m->apart,
+                           NS);
     else
         hipLaunchKernelGGL(attend_split_kernel, dim3(c.n_head, R, NS), dim3(kSplit), 0, m->ctx->stream, m->qkv,
-                           (int64_t)QC, state, c.n_head, c.n_kv, c.n_layer, l, c.max_t, m->rope, m->k8, m->v8, m->ks,
-                           m->vs, m->apart, NS);
+                           (int64_t)QC, state, c.n_head, c.n_kv, c.n_layer, l, c.max_t, m->rope, k8, v8, ks, vs, m->apart,
+                           NS);
     return NS;
 }
 
@@ -914,7 +917,7 @@ int llama_layers(llmq_llama *m, int R, int T, int seq0, int pos0, const int *sta
             fq.in_s = fq.norm = true;
             fq.eps = c.eps;
             RC(launch_gguf_gemm_h16(ctx, m->wqkv[l], m->hs[cur], R, m->qkv, QC, nullptr, 0, &fq));
-            const int NS = attend_splits(m, R, l, state);
+            const int NS = attend_splits(m, R, l, state, seq0);
             uint8_t *pl;
             _Float16 *su;
             float *iv;
@@ -945,7 +948,7 @@ int llama_layers(llmq_llama *m, int R, int T, int seq0, int pos0, const int *sta
         }
         RC(norm_linear(m, gain(m, l, 0), m->wqkv[l], R, m->qkv, QC, 0));
         if (state) {  // RoPE, the cache store and the attention splits in one launch
-            const int NS = attend_splits(m, R, l, state);
+            const int NS = attend_splits(m, R, l, state, seq0);
             if (R == 1 && gguf_gemv_attn_ok(m->wo[l], NS, HD)) {  // Wo combines the splits as it stages its row
                 RC(launch_gguf_gemv(ctx, m->wo[l], nullptr, m->x, nullptr, LLMQ_RESID, nullptr, 0, nullptr, 0.0f, 0,
                                     nullptr, nullptr, m->apart, state, kSplit, NS));
@@ -1048,14 +1051,21 @@ int llama_step(llmq_llama *m, int B) {
 }
 
 // Prefill of sequence seq: T tokens (host) at positions pos0.., then its
-// last token's logits and greedy pick (gen row 0 when state is null).
+// last token's logits and greedy pick (gen row 0 when state is null).  A
+// forward of one token takes the decode step's kernels (RoPE, the store and attention over
+// position splits, combined by Wo), its position uploaded behind the token:
+// the prompt attention's 4 workgroups took 37 us a layer at 400 positions,
+// the splits take 5.5 (a one-token forward 1.7 -> 0.8 ms).
 int llama_prefill(llmq_llama *m, int seq, const int64_t *tokens, int T, int pos0, int B, bool pick) {
     llmq_ctx *ctx = m->ctx;
     const llmq_llama_cfg &c = m->cfg;
     RC(ensure_rows(m, T));
-    LLMQ_HIP(hipMemcpyAsync(m->tokens, tokens, sizeof(int64_t) * T, hipMemcpyHostToDevice, ctx->stream));
+    const bool step = T == 1 && !pick;  // (forward, which waits for the copy of `one` before it returns)
+    const int64_t one[2] = {tokens[0], pos0};
+    LLMQ_HIP(hipMemcpyAsync(m->tokens, step ? one : tokens, sizeof(int64_t) * (step ? 2 : T), hipMemcpyHostToDevice,
+                            ctx->stream));
     RC(launch_gguf_dequant_rows(ctx, m->embd, m->tokens, T, m->x, c.dim));
-    RC(llama_layers(m, T, T, seq, pos0, nullptr));
+    RC(llama_layers(m, T, T, seq, pos0, step ? reinterpret_cast<const int *>(m->tokens + 1) : nullptr));
     RC(llama_head(m, T - 1, 1));
     if (pick)
         hipLaunchKernelGGL(argmax_kernel, dim3(1), dim3(kArgNT), 0, ctx->stream, m->logits, (int64_t)c.vocab, c.vocab,

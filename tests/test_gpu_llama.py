@@ -308,3 +308,33 @@ def test_llama_batch_fused_records_match_numpy(gpu, monkeypatch, B):
         compared.append(n)
     print("llama fused batch records: tokens compared", compared, flush=True)
     assert sum(compared) >= 6 * B, compared
+
+
+@pytest.mark.parametrize("group", [2, 8])
+def test_llama_one_token_forwards_match_numpy(gpu, group):
+    """forward of single tokens (the decode step's split attention) on the
+    second of two sequences, across a split's edge (256 positions) and from
+    an empty cache, against NumPy; the first sequence's cache stays as it
+    was."""
+    torch, lm, ctx = gpu
+    from llm_mojo_amd import synth
+
+    cfg = dict(SMALL, max_t=300, n_head=4 if group == 2 else 8, n_kv=2 if group == 2 else 1,
+               dim=256 if group == 2 else 512)
+    tensors = synth.llama_tensors(cfg, 9, centered=True)
+    toks = synth.llama_prompts(9, 2, 262, cfg["vocab"])
+    m = lm.Llama(ctx, cfg, tensors)
+    ref = NumpyLlama(cfg, tensors, n_seq=2)
+    print("llama one-token forwards", group, flush=True)
+    first = m.forward(0, toks[0][:40], 0)
+    for i in range(3):  # from an empty cache
+        assert rel(m.forward(1, toks[1][i:i + 1], i), ref.forward(1, toks[1][i:i + 1], i)) < 1e-3, i
+    m.forward(1, toks[1][3:254], 3)
+    ref.forward(1, toks[1][3:254], 3)
+    for i in range(254, 262):
+        assert rel(m.forward(1, toks[1][i:i + 1], i), ref.forward(1, toks[1][i:i + 1], i)) < 1e-3, i
+    assert np.array_equal(m.forward(0, toks[0][38:40], 38), m.forward(0, toks[0][38:40], 38))
+    ref.forward(0, toks[0][:40], 0)
+    assert rel(first, ref.forward(0, toks[0][38:40], 38)) < 1e-3
+    assert rel(m.forward(0, toks[0][40:41], 40), ref.forward(0, toks[0][40:41], 40)) < 1e-3
+    m.free()

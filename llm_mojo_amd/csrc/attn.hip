@@ -43,11 +43,21 @@ __global__ __launch_bounds__(64) void kv_store_kernel(const float *__restrict__ 
 // dimension's fma chain over positions (one thread per dimension).
 //
 // The thread that scores position s also copies that position's value row
-// and scale into LDS (STAGE), so the value pass reads no global memory.  With
+// and scale into LDS, so the value pass reads no global memory: MODE 1 as
+// rows, MODE 2 (64 dimensions) as columns, a dimension's positions in one
+// run, for the two serial chains above it (quad_total, pair_values).  With
 // STORE (one token per launch: decode) the workgroup first quantizes its
 // head's new key and value (QuantKV.store, kvcache.mojo:333-342), writes them
 // to the cache, and uses them from LDS for the current position.
-constexpr int kAttnThreads = 256;
+//
+// What bounds it: one workgroup a head, so one CU's latency and the chains'
+// instructions.  MODE 2 against rows with a chain a lane, read by flat loads
+// (s_memtime cycles at 496 positions): total 7500 -> 2600, values 11400 ->
+// 6200, the whole kernel 16.2 -> ~11 us; GPT-2 decode after 476 tokens 410 ->
+// 352 us a token, after 900 541 -> 441, after 12 273 -> 264.  Values as fp16
+// columns for a mixed fma were slower (64 two-byte stores a position), a
+// chain of four lanes' quads too (its broadcast reads fill the LDS port), and
+// so were 10 waves, two of them without positions (the registers spill).
 typedef int v4i __attribute__((ext_vector_type(4)));
 
 // Workgroup barrier ordering LDS only (global loads stay in flight).
@@ -57,31 +67,145 @@ __device__ __forceinline__ void lds_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-template <int HD, bool STAGE, bool STORE>
-__global__ __launch_bounds__(kAttnThreads) void kv_attend_kernel(const float *__restrict__ qkv, int64_t ld, int C,
+// The two serial chains of attend_float_one.  A wave issues an instruction
+// every 4-5 cycles, dependent or not, so a chain costs its instructions, as
+// long as its LDS reads (a latency of ~130 cycles) stay ahead of it: both
+// keep a batch of operands in registers while the next is on its way, and
+// lanes that share a chain each bring a part of the operands, which the add
+// or fma takes from its lane by DPP.  The positions past n, up to a multiple
+// of 16, hold -0.0 (as weights: times codes of 0), which leaves a sum as it
+// is, bit for bit.
+//
+// e[0] + e[1] + ... + e[n - 1] in that order, in every lane: lane q of a quad
+// reads floats 4 q .. of every 16, an add a position.  e is 16-byte aligned.
+#define LLMQ_QADD(r, j) "v_add_f32_dpp %0, %" #r ", %0 quad_perm:[" #j "," #j "," #j "," #j "] row_mask:0xf bank_mask:0xf\n"
+#define LLMQ_QADD4(j) LLMQ_QADD(1, j) LLMQ_QADD(2, j) LLMQ_QADD(3, j) LLMQ_QADD(4, j)
+typedef float v4fa __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ float quad_total(const float *e, int n) {
+    const v4fa *p = reinterpret_cast<const v4fa *>(e) + (threadIdx.x & 3);
+    float t = 0.0f;
+    v4fa a[4], b[4];
+    auto load = [&](v4fa (&x)[4], int s) {
+#pragma unroll
+        for (int k = 0; k < 4; k++) x[k] = p[s / 4 + 4 * k];
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto add16 = [&](const v4fa &x) {
+        asm volatile("s_nop 1\n" LLMQ_QADD4(0) LLMQ_QADD4(1) LLMQ_QADD4(2) LLMQ_QADD4(3)
+                     : "+v"(t)
+                     : "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]));
+    };
+    auto add = [&](const v4fa (&x)[4], int s) {
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+            if (s + 16 * k < n) add16(x[k]);
+    };
+    load(a, 0);
+    for (int s = 0; s < n; s += 128) {
+        load(b, s + 64);
+        add(a, s);
+        if (s + 64 >= n) break;
+        load(a, s + 128);
+        add(b, s + 64);
+    }
+    return t;
+}
+#undef LLMQ_QADD4
+#undef LLMQ_QADD
+// acc = fma(w[s], v[s], acc) for s = 0 .. n - 1 from 0, in both lanes of a
+// pair: lane h of it reads the codes v of 8 h .. of every 16 positions (v:
+// the pair's dimension, its positions in one run) and converts them.
+#define LLMQ_CODE(f, c, b) \
+    asm("v_cvt_f32_i32_sdwa %0, sext(%1) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_" #b : "=v"(f) : "v"(c))
+#define LLMQ_PFMA(f, w, h) "v_fmac_f32_dpp %0, %" #f ", %" #w " quad_perm:[" h "] row_mask:0xf bank_mask:0xf\n"
+#define LLMQ_PFMA4(f0, f1, f2, f3, w0, w1, w2, w3, h) \
+    LLMQ_PFMA(f0, w0, h) LLMQ_PFMA(f1, w1, h) LLMQ_PFMA(f2, w2, h) LLMQ_PFMA(f3, w3, h)
+__device__ __forceinline__ float pair_values(const float *w, const int8_t *v, int n) {
+    typedef uint32_t v2ua __attribute__((ext_vector_type(2)));
+    const v4fa *wp = reinterpret_cast<const v4fa *>(w);
+    const v2ua *vp = reinterpret_cast<const v2ua *>(v) + (threadIdx.x & 1);
+    float acc = 0.0f;
+    struct Batch {
+        v4fa w[8];
+        v2ua c[2];
+    } a, b;
+    auto load = [&](Batch &x, int s) {
+#pragma unroll
+        for (int k = 0; k < 8; k++) x.w[k] = wp[s / 4 + k];
+#pragma unroll
+        for (int k = 0; k < 2; k++) x.c[k] = vp[s / 8 + 2 * k];
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto add16 = [&](const v4fa *x, v2ua c) {
+        float f[8];
+#pragma unroll
+        for (int k = 0; k < 2; k++) {  // one instruction a code (written in C, a shift and a sign extension as well)
+            LLMQ_CODE(f[4 * k], c[k], 0);
+            LLMQ_CODE(f[4 * k + 1], c[k], 1);
+            LLMQ_CODE(f[4 * k + 2], c[k], 2);
+            LLMQ_CODE(f[4 * k + 3], c[k], 3);
+        }
+        asm volatile("s_nop 1\n" LLMQ_PFMA4(1, 2, 3, 4, 9, 10, 11, 12, "0,0,2,2") LLMQ_PFMA4(5, 6, 7, 8, 13, 14, 15, 16, "0,0,2,2")
+                         LLMQ_PFMA4(1, 2, 3, 4, 17, 18, 19, 20, "1,1,3,3") LLMQ_PFMA4(5, 6, 7, 8, 21, 22, 23, 24, "1,1,3,3")
+                     : "+v"(acc)
+                     : "v"(f[0]), "v"(f[1]), "v"(f[2]), "v"(f[3]), "v"(f[4]), "v"(f[5]), "v"(f[6]), "v"(f[7]),
+                       "v"(x[0][0]), "v"(x[0][1]), "v"(x[0][2]), "v"(x[0][3]), "v"(x[1][0]), "v"(x[1][1]), "v"(x[1][2]),
+                       "v"(x[1][3]), "v"(x[2][0]), "v"(x[2][1]), "v"(x[2][2]), "v"(x[2][3]), "v"(x[3][0]), "v"(x[3][1]),
+                       "v"(x[3][2]), "v"(x[3][3]));
+    };
+    auto add = [&](const Batch &x, int s) {
+        add16(x.w, x.c[0]);
+        if (s + 16 < n) add16(x.w + 4, x.c[1]);
+    };
+    load(a, 0);
+    for (int s = 0; s < n; s += 64) {
+        load(b, s + 32);
+        add(a, s);
+        if (s + 32 >= n) break;
+        load(a, s + 64);
+        add(b, s + 32);
+    }
+    return acc;
+}
+#undef LLMQ_PFMA4
+#undef LLMQ_PFMA
+#undef LLMQ_CODE
+// Entries past max_t that the chains may read ahead of their end, and the
+// bytes of a dimension's codes in LDS: 64 more than a multiple of 128, so
+// that the quads' stores of four dimensions go to different banks.
+constexpr int kAttendPad = 144;
+__host__ __device__ constexpr int attend_vstride(int max_t) { return (max_t + kAttendPad - 64 + 127) / 128 * 128 + 64; }
+
+template <int HD, int MODE, bool STORE, int NT>
+__global__ __launch_bounds__(NT) void kv_attend_kernel(const float *__restrict__ qkv, int64_t ld, int C,
                                                                  int pos0, const int *__restrict__ pos_dev,
                                                                  int layer, int max_t, int n_head,
                                                                  int8_t *__restrict__ K8, int8_t *__restrict__ V8,
                                                                  float *__restrict__ KS, float *__restrict__ VS,
                                                                  float *__restrict__ out, int64_t ldo) {
+    constexpr bool STAGE = MODE != 0, COLS = MODE == 2;
+    static_assert(!COLS || HD == 64, "a pair of lanes a dimension");
     constexpr int NV = HD / 16;  // 16-byte pieces of a row
     extern __shared__ __align__(16) float sm[];
     float *q = sm;                // [HD]
     float *scores = q + HD;       // [max_t]
-    float *vsc = scores + max_t;  // [max_t]  value scales (STAGE)
-    // [max_t][HD] value codes (STAGE), 16-byte aligned for the int4 copies
-    int8_t *vrow = reinterpret_cast<int8_t *>((reinterpret_cast<uintptr_t>(vsc + max_t) + 15) & ~(uintptr_t)15);
-    __shared__ float red[kAttnThreads];
+    float *vsc = scores + max_t + (COLS ? kAttendPad : 0);  // [max_t]  value scales (STAGE)
+    // the value codes, 16-byte aligned (by an offset: through an integer the
+    // pointer would lose its address space, and every read be a flat load):
+    // rows [max_t][HD], or (COLS) columns [HD][attend_vstride]
+    int8_t *vrow = reinterpret_cast<int8_t *>(sm) + (((HD + 2 * max_t + (COLS ? kAttendPad : 0)) * 4 + 15) & ~15);
+    const int vst = attend_vstride(max_t);
+    __shared__ float red[NT / 64];
     __shared__ __align__(16) int8_t knew[HD], vnew[HD];
     __shared__ float kscale_new, vscale_new;
     const int h = blockIdx.x, t = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-    const int npos = (pos_dev ? *pos_dev : pos0) + t + 1;
-    const int cur = npos - 1;
     const float scale = 1.0f / sqrtf((float)HD);
     const int64_t base = (int64_t)layer * max_t * n_head + h;  // slot of position 0
 
     // The rows of this thread's first position, requested before anything
-    // else (positions past the end re-read the last one and are not used).
+    // else: those of the first waves without waiting for the position, the
+    // others within it (past the end they re-read the last one; not used).
+    constexpr int kEarly = 1;
     v4i kr[NV], vr[NV];  // native vectors: HIP's int4 struct copies kept vr in scratch
     float ksr, vsr;
     auto load_row = [&](int s) {
@@ -96,13 +220,20 @@ __global__ __launch_bounds__(kAttnThreads) void kv_attend_kernel(const float *__
         ksr = KS[sl];
         if (STAGE) vsr = VS[sl];
     };
-    load_row(tid < npos ? tid : cur);
+    if (wid < kEarly) load_row(min(tid, max_t - 1));
+    __builtin_amdgcn_sched_barrier(0);
+    const int npos = (pos_dev ? *pos_dev : pos0) + t + 1;
+    const int cur = npos - 1;
+    if (wid >= kEarly && wid * 64 < npos) load_row(min(tid, cur));
     __builtin_amdgcn_sched_barrier(0);
 
-    for (int i = tid; i < HD; i += kAttnThreads) q[i] = qkv[(int64_t)t * ld + (int64_t)h * HD + i];
-    if (STORE && (wid == 1 || wid == 2)) {
+    // (the query and the new rows by waves whose own rows, if any, were not requested ahead of them)
+    constexpr int NW = NT / 64;
+    if (wid == NW - 4)
+        for (int i = lane; i < HD; i += 64) q[i] = qkv[(int64_t)t * ld + (int64_t)h * HD + i];
+    if (STORE && (wid == NW - 3 || wid == NW - 2)) {
         // QuantKV.store for this head (kvcache.mojo:320-342)
-        const int kv = wid - 1;
+        const int kv = wid - (NW - 3);
         const float *src = qkv + (int64_t)t * ld + (int64_t)(1 + kv) * C + (int64_t)h * HD;
         float xs[HD / 64];
         float m = 0.0f;
@@ -125,7 +256,7 @@ __global__ __launch_bounds__(kAttnThreads) void kv_attend_kernel(const float *__
             // back from global memory.
             if (kv == 0)
                 knew[i] = code;
-            else if (STAGE)
+            else if (STAGE && !COLS)
                 vrow[(int64_t)cur * HD + i] = code;
             else
                 vnew[i] = code;
@@ -142,10 +273,31 @@ __global__ __launch_bounds__(kAttnThreads) void kv_attend_kernel(const float *__
     }
     lds_barrier();
 
+    // The value codes vr of a quad's four positions to columns, transposed by
+    // bytes: lane q keeps dimension 4 e + q of each dword e (0 past the end).
+    // A wave's last rows wait until the last wave, which has none before
+    // position 448, forms the total.
+    int later = -1;
+    auto columns = [&](int s, bool live) {
+        if (STORE && s == cur) {
+#pragma unroll
+            for (int i = 0; i < NV; i++) vr[i] = *reinterpret_cast<const v4i *>(vnew + 16 * i);
+        }
+        const uint32_t s1 = (lane & 1) ? 0x07030501u : 0x02060004u, s2 = (lane & 2) ? 0x03020706u : 0x05040100u;
+        int8_t *o = vrow + (lane & 3) * vst + (s & ~3);
+#pragma unroll
+        for (int e = 0; e < 4 * NV; e++) {
+            const uint32_t x = live ? (uint32_t)vr[e / 4][e % 4] : 0u;
+            const uint32_t y = __builtin_amdgcn_perm(x, (uint32_t)llmq_dppi<0xB1>((int)x), s1);
+            const uint32_t z = __builtin_amdgcn_perm((uint32_t)llmq_dppi<0x4E>((int)y), y, s2);
+            *reinterpret_cast<uint32_t *>(o + 4 * e * vst) = z;
+        }
+    };
     float mx = -INFINITY;
-    for (int s = tid; s < npos; s += kAttnThreads) {
-        if (s != tid) load_row(s);  // only past 256 positions
-        const bool fresh = STORE && s == cur;
+    const int nend = COLS ? (npos + 15) & ~15 : npos;
+    for (int s = tid; s < nend; s += NT) {
+        if (s != tid) load_row(min(s, cur));  // only past NT positions
+        const bool fresh = STORE && s == cur, live = !COLS || s < npos;
         if (fresh) {
 #pragma unroll
             for (int i = 0; i < NV; i++) kr[i] = *reinterpret_cast<const v4i *>(knew + 16 * i);
@@ -170,26 +322,56 @@ __global__ __launch_bounds__(kAttnThreads) void kv_attend_kernel(const float *__
         dl[0] = dl[0] + dl[2];
         dl[1] = dl[1] + dl[3];
         const float d = dl[0] + dl[1];
-        if (STAGE && !fresh) {
+        if constexpr (COLS) {
+            if (live && !fresh) vsc[s] = vsr;
+            if (wid == NW - 1 || s + NT < nend)
+                columns(s, live);
+            else
+                later = s;
+        } else if (STAGE && !fresh) {
 #pragma unroll
             for (int i = 0; i < NV; i++) *reinterpret_cast<v4i *>(vrow + (int64_t)s * HD + 16 * i) = vr[i];
             vsc[s] = vsr;
         }
         const float sc = (d * ksr) * scale;
-        scores[s] = sc;
-        mx = fmaxf(mx, sc);
+        if (live) {
+            scores[s] = sc;
+            mx = fmaxf(mx, sc);
+        }
     }
     mx = wave_max(mx);
     if ((tid & 63) == 0) red[tid >> 6] = mx;
     lds_barrier();
-    mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-    for (int s = tid; s < npos; s += kAttnThreads) scores[s] = ref_expf(scores[s] - mx);
+    mx = red[0];
+#pragma unroll
+    for (int i = 1; i < NT / 64; i++) mx = fmaxf(mx, red[i]);
+    for (int s = tid; s < nend; s += NT) scores[s] = s < npos ? ref_expf(scores[s] - mx) : -0.0f;
     lds_barrier();
     auto vscale = [&](int s) -> float {
         if (STAGE) return vsc[s];
         if (STORE && s == cur) return vscale_new;
         return VS[base + (int64_t)s * n_head];
     };
+    if constexpr (COLS) {
+        // The last wave forms the total, the threads turn the positions into
+        // weights, waves 0 and 1 run 32 value chains each.
+        if (wid == NW - 1) {
+            const float sum = quad_total(scores, npos);
+            if (lane == 0) red[0] = sum;
+        } else if (later >= 0) {
+            columns(later, later < npos);
+        }
+        lds_barrier();
+        const float total = red[0];
+        for (int s = tid; s < npos; s += NT) scores[s] = (scores[s] / total) * vsc[s];
+        lds_barrier();
+        if (wid < 2) {
+            const int dim = wid * 32 + (lane >> 1);
+            const float acc = pair_values(scores, vrow + dim * vst, npos);
+            if ((lane & 1) == 0) out[(int64_t)t * ldo + (int64_t)h * HD + dim] = acc;
+        }
+        return;
+    }
     // The total in position order (attend_float_one, 139-141): 16 scores per
     // batch of LDS reads, then their adds in order.
     auto total_of = [&]() -> float {
@@ -246,7 +428,7 @@ __global__ __launch_bounds__(kAttnThreads) void kv_attend_kernel(const float *__
         if (tid == 0) red[0] = total_of();
         lds_barrier();
         const float total = red[0];
-        for (int s = tid; s < npos; s += kAttnThreads) scores[s] = (scores[s] / total) * vscale(s);
+        for (int s = tid; s < npos; s += NT) scores[s] = (scores[s] / total) * vscale(s);
         lds_barrier();
         if (tid < HD) out[(int64_t)t * ldo + (int64_t)h * HD + tid] = value_chain(tid);
     }
@@ -1104,11 +1286,11 @@ int launch_kv_store(llmq_ctx *ctx, llmq_kv *kv, int layer, int pos0, const int *
     return LLMQ_OK;
 }
 
-template <int HD, bool STAGE, bool STORE>
+template <int HD, int MODE, bool STORE, int NT>
 static int attend_launch(llmq_ctx *ctx, const llmq_kv *kv, float *out, const float *qkv, int layer, int T, int pos0,
                          const int *pos_dev, int64_t ld, size_t lds) {
     const int C = kv->n_head * kv->head_dim;
-    hipLaunchKernelGGL((kv_attend_kernel<HD, STAGE, STORE>), dim3(kv->n_head, T), dim3(kAttnThreads), lds, ctx->stream,
+    hipLaunchKernelGGL((kv_attend_kernel<HD, MODE, STORE, NT>), dim3(kv->n_head, T), dim3(NT), lds, ctx->stream,
                        qkv, ld ? ld : 3 * C, C, pos0, pos_dev, layer, kv->max_t, kv->n_head, kv->k, kv->v, kv->ks,
                        kv->vs, out, (int64_t)C);
     LLMQ_HIP(hipGetLastError());
@@ -1117,11 +1299,11 @@ static int attend_launch(llmq_ctx *ctx, const llmq_kv *kv, float *out, const flo
 
 // Raises a kernel's dynamic LDS limit to `bytes` once; false if the device
 // does not allow that much.
-template <int HD, bool STAGE, bool STORE>
+template <int HD, int MODE, bool STORE, int NT>
 static bool allow_lds(size_t bytes) {
     static size_t granted = 64 * 1024;
     if (bytes <= granted) return true;
-    if (hipFuncSetAttribute(reinterpret_cast<const void *>(&kv_attend_kernel<HD, STAGE, STORE>),
+    if (hipFuncSetAttribute(reinterpret_cast<const void *>(&kv_attend_kernel<HD, MODE, STORE, NT>),
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) != hipSuccess) {
         (void)hipGetLastError();
         return false;
@@ -1130,17 +1312,19 @@ static bool allow_lds(size_t bytes) {
     return true;
 }
 
-template <int HD>
+template <int HD, bool STORE>
 static int attend_hd(llmq_ctx *ctx, const llmq_kv *kv, float *out, const float *qkv, int layer, int T, int pos0,
-                     const int *pos_dev, int64_t ld, bool store) {
+                     const int *pos_dev, int64_t ld) {
     const size_t base = sizeof(float) * ((size_t)HD + kv->max_t);
-    const size_t staged = base + (size_t)kv->max_t * (sizeof(float) + HD) + 16;
-    if (store && allow_lds<HD, true, true>(staged))
-        return attend_launch<HD, true, true>(ctx, kv, out, qkv, layer, T, pos0, pos_dev, ld, staged);
-    if (!store && allow_lds<HD, true, false>(staged))
-        return attend_launch<HD, true, false>(ctx, kv, out, qkv, layer, T, pos0, pos_dev, ld, staged);
-    return store ? attend_launch<HD, false, true>(ctx, kv, out, qkv, layer, T, pos0, pos_dev, ld, base)
-                 : attend_launch<HD, false, false>(ctx, kv, out, qkv, layer, T, pos0, pos_dev, ld, base);
+    const size_t rows = base + (size_t)kv->max_t * (sizeof(float) + HD) + 16;
+    if constexpr (HD == 64) {
+        const size_t cols = base + sizeof(float) * ((size_t)kv->max_t + kAttendPad) + 16 + (size_t)HD * attend_vstride(kv->max_t);
+        if (allow_lds<HD, 2, STORE, 512>(cols))
+            return attend_launch<HD, 2, STORE, 512>(ctx, kv, out, qkv, layer, T, pos0, pos_dev, ld, cols);
+    }
+    if (allow_lds<HD, 1, STORE, 256>(rows))
+        return attend_launch<HD, 1, STORE, 256>(ctx, kv, out, qkv, layer, T, pos0, pos_dev, ld, rows);
+    return attend_launch<HD, 0, STORE, 256>(ctx, kv, out, qkv, layer, T, pos0, pos_dev, ld, base);
 }
 
 // The exact-order prompt attention (head_dim 64); LLMQ_PROMPT_NTH /
@@ -1194,8 +1378,12 @@ int launch_kv_attend(llmq_ctx *ctx, const llmq_kv *kv, float *out, const float *
         if (sv && sv[0] == '0') return prompt_exact_launch<512, 16, false>(ctx, kv, out, qkv, layer, T, pos0, ld);
         return prompt_exact_launch<512, 16, true>(ctx, kv, out, qkv, layer, T, pos0, ld);
     }
-    if (kv->head_dim == 64) return attend_hd<64>(ctx, kv, out, qkv, layer, T, pos0, pos_dev, ld, store);
-    if (kv->head_dim == 128) return attend_hd<128>(ctx, kv, out, qkv, layer, T, pos0, pos_dev, ld, store);
+    if (kv->head_dim == 64)
+        return store ? attend_hd<64, true>(ctx, kv, out, qkv, layer, T, pos0, pos_dev, ld)
+                     : attend_hd<64, false>(ctx, kv, out, qkv, layer, T, pos0, pos_dev, ld);
+    if (kv->head_dim == 128)
+        return store ? attend_hd<128, true>(ctx, kv, out, qkv, layer, T, pos0, pos_dev, ld)
+                     : attend_hd<128, false>(ctx, kv, out, qkv, layer, T, pos0, pos_dev, ld);
     return llmq_set_error(LLMQ_EUNSUPPORTED, "kv_attend: head_dim %d (64 or 128)", kv->head_dim);
 }
 

@@ -183,9 +183,10 @@ LLMQ_API int llmq_linear(llmq_ctx *ctx, float *out, const float *x, const llmq_m
  * hipFree.  Sizes needing more scratch than that (a16: T x IN x 2 bytes
  * and T x 4, each rounded up to 256; Q4_K: the record's ~4.4 x T x IN
  * bytes, T rounded up to 16) return LLMQ_EINVAL; other float-activation
- * formats take as many tokens at a time as the scratch holds.  An int4-g32 a16 matrix also puts its prompt GEMM's fp16
- * activation planes there (T x IN x 4 bytes, T rounded up to 16) when they
- * fit, else runs the int8-MFMA form of the same GEMM (the same bits).
+ * formats take as many tokens at a time as the scratch holds.  An a16 matrix
+ * in groups of 32, or of whole 256-input superblocks, also puts its prompt
+ * GEMM's fp16 activation planes there (T x IN x 4 bytes, T rounded up to 16)
+ * when they fit, else runs the int8-MFMA form of the GEMM (the same bits).
  * Every call on one GPU shares the array: calls that overlap in time on one
  * GPU (different streams or threads) race; calls ordered on one stream do
  * not.  Nothing in the scratch needs to start at zero (each call writes all

@@ -410,6 +410,13 @@ int gemm_planes_tile(const llmq_mat *w, int64_t T);
 int launch_gemm_planes(llmq_ctx *ctx, const llmq_mat *w, const void *rec, int64_t T, float *out, int64_t ldo,
                        const float *bias, int flags, int tile);
 // (rows: a wave a superblock of a token, for one token tile of Q4_K)
+// The same kernel over int16 activation codes as fp16 planes (gemm_mfma.hip's
+// layout; sx the tokens' scales): the first n rows of w, whose K is whole
+// superblocks and whose groups are a power of two times 32 or the row; the
+// bits are tile_i16's.
+bool gemm_planes_a16_ok(const llmq_mat *w);
+int launch_gemm_planes_a16(llmq_ctx *ctx, const llmq_mat *w, const uint8_t *pl, const float *sx, int64_t T, int64_t n,
+                           float *out, int64_t ldo, const float *bias, int flags);
 int launch_act_h16(llmq_ctx *ctx, const float *x, int64_t ldx, int64_t T, int64_t K, void *rec, bool rows = false);
 // The batch-decode chain's forms of that matmul (gguf_gemm16.hip): the
 // input may be an "h16s" record (a scale per 16 inputs of a token, written

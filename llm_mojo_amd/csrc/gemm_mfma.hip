@@ -40,9 +40,12 @@
 // instructions (per-workgroup timestamps), and prefetching four blocks
 // ahead instead of two does not shorten it.
 //
-// int4 weights in groups of 32 take gemm_f16_kernel instead (below): the
-// same G on the fp16 matrix cores, exact in their fp32 sums, so the flush is
-// one fma per output and group.
+// Where the activations' fp16 planes fit the workspace, groups of 32 take
+// gemm_f16_kernel instead (below), and matrices of whole 256-input
+// superblocks gemm_planes.hip's kernel: the same G on the fp16 matrix cores,
+// exact in their fp32 sums, so the flush is one fma per output and group
+// (301 tokens of 3072 x 768 int8 per channel: 32.4 -> 20.6 us with the
+// activations; 512 of 4096 x 4096 109 -> 59).
 //
 // Activations come from act_q16_kernel: LayerNorm (kernels.mojo:179-197) when
 // asked, then quantize_rows (kernels.mojo:400-416), one workgroup per token.
@@ -803,7 +806,7 @@ bool gemm_mfma_supports(const llmq_mat *w, int64_t T) {
 bool gemm_f16_supports(const llmq_mat *w, int64_t T) {
     if (const char *e = getenv("LLMQ_MFMA_F16"))
         if (atoi(e) == 0) return false;
-    return gemm_mfma_supports(w, T) && (w->bits == 4 || w->bits == 8) && w->group == 32 &&
+    return gemm_mfma_supports(w, T) && (w->bits == 4 || w->bits == 8) && (w->group == 32 || gemm_planes_a16_ok(w)) &&
            (T + 15) / 16 * 16 * w->k * 4 < (int64_t)kOOB;
 }
 
@@ -818,7 +821,7 @@ bool gemm_kv_fold_ok(const llmq_mat *w, int64_t T, const llmq_kv *cache) {
     if (getenv("LLMQ_MFMA_MIN_T")) return false;
     if (!cache || cache->integer || cache->head_dim != 64 || T < min_t || !w->a16) return false;
     const int64_t C = (int64_t)cache->n_head * 64;
-    return gemm_f16_supports(w, T) && w->n == 3 * C && w->n % 64 == 0;
+    return gemm_f16_supports(w, T) && w->group == 32 && w->n == 3 * C && w->n % 64 == 0;
 }
 
 int launch_gemm_mfma(llmq_ctx *ctx, const GemvRequest &rq, int16_t *xq, float *sx, uint8_t *planes) {
@@ -848,7 +851,15 @@ int launch_gemm_mfma(llmq_ctx *ctx, const GemvRequest &rq, int16_t *xq, float *s
     // the 32-row tiles; the rest (n % 32 rows: the vocabulary's last 17)
     // go through rows_i16 below
     const int full = (int)(w->n / 32 * 32);
-    if (planes && full > 0) {
+    // gemm_planes.hip's tiles, except where the 16 x 64 tile of
+    // gemm_f16_kernel is the faster one: int4 in groups of 32 with fewer than
+    // 640 workgroups of 32 x 64 (301 x 3072 x 768 21.2 us here, 23.3 there;
+    // 476 x 768 x 3072 15.9 and 14.8; int8 27.9 and 23.3, 18.6 and 17.6)
+    const bool big = (T + 31) / 32 * ((full + 63) / 64) >= 640;
+    if (planes && full > 0 && !rq.kv && gemm_planes_a16_ok(w) && !(w->group == 32 && getenv("LLMQ_F16_TILE")) &&
+        (w->group != 32 || w->bits == 8 || big)) {
+        RC(launch_gemm_planes_a16(ctx, w, planes, sx, T, full, rq.out, rq.ldo ? rq.ldo : w->n, rq.bias, rq.flags));
+    } else if (planes && full > 0) {
         F16Args f;
         f.planes = planes;
         f.codes = w->codes;

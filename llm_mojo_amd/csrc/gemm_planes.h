@@ -39,6 +39,13 @@
 // 512 x 4096 x 11008: Q8_0 1058 us on the fp32 matrix cores, 126 here
 // (0.73 PFLOP/s of fp16 products); Q6_K 1175 -> 160, Q5_K 777 -> 148,
 // Q4_0 1137 -> 115, Q4_1 1135 -> 135, int8-ch 1147 -> 114.
+//
+// int16 activation codes (kA4, kA8) come as two exact planes of their own,
+// 256 hi + lo: every partial sum of a segment (at most 256 inputs) is a whole
+// number below 2^24, so hi + lo is the integer and one fma per output and
+// segment, in the reference's order, gives the int8 matrix cores' bits
+// (512 x 4096 x 4096 with the activations: int8-ch 109 -> 59 us, int4-ch
+// 72 -> 57, int8-g32 88 -> 70).
 #pragma once
 #include <type_traits>
 
@@ -50,7 +57,7 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef _Float16 v2h __attribute__((ext_vector_type(2)));
 
-enum Fmt { kQ8_0, kQ4_0, kQ4_1, kQ4_K, kQ5_K, kQ6_K, kQm4, kQm8 };
+enum Fmt { kQ8_0, kQ4_0, kQ4_1, kQ4_K, kQ5_K, kQ6_K, kQm4, kQm8, kA4, kA8 };
 
 struct Args {
     const uint8_t *planes, *sums, *inv;        // the h16 record
@@ -58,7 +65,7 @@ struct Args {
     int T, n, ntiles, NC, NSB, NG, gshift, flags;  // NC chunks of 32 inputs, NSB superblocks, NG groups a row
     int rows_first;                                // workgroup order: row blocks fastest
     int64_t ldo;
-    const float *bias;
+    const float *bias, *sx;  // sx: the tokens' scales (A16)
     float *out;
 };
 
@@ -66,8 +73,9 @@ struct Args {
 template <int F>
 struct Tr {
     static constexpr bool KQ = F == kQ4_K || F == kQ5_K || F == kQ6_K;
-    static constexpr bool QM = F == kQm4 || F == kQm8;
-    static constexpr bool W8 = F == kQ8_0 || F == kQm8;
+    static constexpr bool A16 = F == kA4 || F == kA8;                       // int16 activation codes
+    static constexpr bool QM = F == kQm4 || F == kQm8 || A16;
+    static constexpr bool W8 = F == kQ8_0 || F == kQm8 || F == kA8;
     static constexpr int CB = W8 ? 512 : 256;                               // codes
     static constexpr int SCB = KQ ? 0 : F == kQ4_1 ? 64 : 32;               // scales
     static constexpr int ZB = QM ? 16 : 0;                                  // zero points
@@ -102,7 +110,7 @@ struct Lay {
     static constexpr int A = NTT * S * 2048, C = NRT * S * R::CB, SC = NRT * S * R::SCB, Z = NRT * S * R::ZB,
                          H = NRT * S * R::HB;
     static constexpr int oC = A, oSC = oC + C, oZ = oSC + SC, oH = oZ + Z, STEP = oH + H;
-    static constexpr int SBF = NRT * R::SBF, SBD = NRT * R::SBD, SU = R::SUMS ? NTT * 512 : 0, IV = NTT * 64;
+    static constexpr int SBF = NRT * R::SBF, SBD = NRT * R::SBD, SU = R::SUMS ? NTT * 512 : 0, IV = R::A16 ? 0 : NTT * 64;
     static constexpr int oSBD = SBF, oSU = oSBD + SBD, oIV = oSU + SU, SBUF = oIV + IV;
 };
 
@@ -117,9 +125,9 @@ __global__ __launch_bounds__(WT * WR * WK * 64, 2) void gemm_planes_kernel(Args 
     constexpr int NW = WT * WR * WK, RB = NW * 1024;  // bytes a copy round: 16 a lane
     // (waves that share a group's chunks scale each by itself)
     constexpr int SEG = WK > 1 && SEG0 < 8 ? 1 : SEG0;
-    constexpr bool CHAIN = R::KQ || SEG == 8;    // one scale a superblock: the products of all 8 chunks chain
+    constexpr bool CHAIN = !R::A16 && (R::KQ || SEG == 8);    // one scale a superblock: the products of all 8 chunks chain
     // separate arrays, so that the compiler sees a copy into one cannot alias reads of another
-    __shared__ __align__(16) uint8_t b0[L::STEP], b1[L::STEP], f0[L::SBUF], f1[L::SBUF];
+    __shared__ __align__(16) uint8_t b0[L::STEP], b1[L::STEP], f0[L::SBUF ? L::SBUF : 16], f1[L::SBUF ? L::SBUF : 16];
     const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int c16 = lane & 15, g = lane >> 4;
     const int wt = w / WR % WT, wr = w % WR, kk = w / (WT * WR);
@@ -204,7 +212,7 @@ __global__ __launch_bounds__(WT * WR * WK * 64, 2) void gemm_planes_kernel(Args 
         const int x = off(LLMQ_N(L::SU), 0);
         vU[0] = ttile(x / 512) * a.NSB * 512 + x % 512;
     }
-    {
+    if constexpr (L::IV > 0) {
         const int x = off(LLMQ_N(L::IV), 0);
         vI[0] = ttile(x / 64) * a.NSB * 64 + x % 64;
     }
@@ -234,7 +242,7 @@ __global__ __launch_bounds__(WT * WR * WK * 64, 2) void gemm_planes_kernel(Args 
         if constexpr (R::SBF > 0) LLMQ_CP(a.sb, buf, L::SBF, vF, sb * 256);
         if constexpr (R::SBD > 0) LLMQ_CP(a.sbd, buf + L::oSBD, L::SBD, vD, sb * 32);
         if constexpr (R::SUMS) LLMQ_CP(a.sums, buf + L::oSU, L::SU, vU, sb * 512);
-        LLMQ_CP(a.inv, buf + L::oIV, L::IV, vI, sb * 64);
+        if constexpr (L::IV > 0) LLMQ_CP(a.inv, buf + L::oIV, L::IV, vI, sb * 64);
     };
 #undef LLMQ_CP
     const v4f zero = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -243,7 +251,7 @@ __global__ __launch_bounds__(WT * WR * WK * 64, 2) void gemm_planes_kernel(Args 
     for (int t = 0; t < TT; t++)
 #pragma unroll
         for (int r = 0; r < RT; r++) acc[t][r] = zero;
-    v4f seg[TT][RT];                // SEG 2, 4: the group's sums
+    v4f seg[TT][RT], sel[TT][RT];   // SEG > 1: the group's sums (A16: of the hi and the lo plane)
     v2h sc[RT][4];                  // K quants: sub-block scales (sc_2i, sc_2i+1); Q6_K: from LDS
     uint32_t mp[RT][4];             // Q4_K: minima of the 8 chunks, fp16 pairs
     float cm[RT][2] = {};           // CENTER: the offsets of chunks g and 4 + g
@@ -395,6 +403,34 @@ __global__ __launch_bounds__(WT * WR * WK * 64, 2) void gemm_planes_kernel(Args 
                     if ((j + WK) % SEG == 0) s = h2f(lds<uint16_t>(cur, pS + e * 32));
                     if (SEG == 8 && j + WK == 8) rs[r] = s;
                 }
+                if constexpr (R::A16) {
+                    // sum 256 hi w and sum lo w over the group's chunks (256 inputs at most), each exact
+                    // (multiples of 256 below 2^32, whole numbers below 2^24), and their one rounded sum
+                    // float(G); int4 in groups of 32: |G| < 2^24, one exact chain
+                    constexpr bool one = F == kA4 && SEG == 1;
+                    v4f xh[TT], xl[TT];
+#pragma unroll
+                    for (int t = 0; t < TT; t++)
+                        xh[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, ah[t]), b,
+                                                                       j % SEG == 0 ? zero : seg[t][r], 0, 0, 0);
+#pragma unroll
+                    for (int t = 0; t < TT; t++)
+                        xl[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                            __builtin_bit_cast(v8h, al[t]), b, one ? xh[t] : j % SEG == 0 ? zero : sel[t][r], 0, 0, 0);
+#pragma unroll
+                    for (int t = 0; t < TT; t++) {
+                        if ((j + 1) % SEG == 0) {  // tile_i16's flush
+#pragma unroll
+                            for (int i = 0; i < 4; i++)
+                                acc[t][r][i] = fmaf(one ? xl[t][i] : xh[t][i] + xl[t][i], s, acc[t][r][i]);
+                            asm volatile("" : "+v"(acc[t][r]));  // (formed here, as in scale())
+                        } else {
+                            seg[t][r] = xh[t];
+                            sel[t][r] = xl[t];
+                        }
+                    }
+                    continue;
+                }
                 v4f x[TT];
 #pragma unroll
                 for (int t = 0; t < TT; t++) {
@@ -424,7 +460,7 @@ __global__ __launch_bounds__(WT * WR * WK * 64, 2) void gemm_planes_kernel(Args 
                 }
             }
         }
-        if constexpr (j0 + S == 8) {  // the superblock's minima, scale and 1 / s
+        if constexpr (j0 + S == 8 && !R::A16) {  // the superblock's minima, scale and 1 / s
             float dd[RT], dmin[RT];
             v8h bm[RT];
 #pragma unroll
@@ -546,6 +582,7 @@ __global__ __launch_bounds__(WT * WR * WK * 64, 2) void gemm_planes_kernel(Args 
                 const int tok = (tt0 + wt * TT + t) * 16 + 4 * g + i;
                 if (!rok || tok >= a.T) continue;
                 float v = acc[t][r][i];
+                if constexpr (R::A16) v *= a.sx[tok];
                 if (a.flags & LLMQ_BIAS) v += bo;
                 if (a.flags & LLMQ_GELU) v = gelu_ref(v);
                 float *dst = a.out + (int64_t)tok * a.ldo + o;
@@ -564,6 +601,16 @@ int launch_tile(hipStream_t st, int tile, const Args &a) {
     hipLaunchKernelGGL((gemm_planes_kernel<F, SEG, TT, RT, WT, WR, WK, S>),                                     \
                        dim3((unsigned)((rt + WR * RT - 1) / (WR * RT)), (unsigned)((tt + WT * TT - 1) / (WT * TT))), \
                        dim3(WT *WR * WK * 64), 0, st, a)
+    if constexpr (Tr<F>::A16) {  // the segments' fma order is the reference's: no tiles that split the axis
+        switch (tile) {
+        case 1: LLMQ_PK(2, 4, 2, 2, 1, 2); break;
+        case 2: LLMQ_PK(2, 2, 2, 2, 1, 2); break;
+        case 3: LLMQ_PK(2, 1, 1, 4, 1, 4); break;
+        default: LLMQ_PK(1, 1, 1, 4, 1, 4); break;
+        }
+        LLMQ_HIP(hipGetLastError());
+        return LLMQ_OK;
+    } else
     switch (tile) {
     case 0:  // (only where the registers hold it: one scale a superblock)
         if constexpr (SEG == 8)

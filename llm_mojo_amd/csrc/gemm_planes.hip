@@ -8,6 +8,8 @@ namespace planes {
 LLMQ_PX(kQ8_0, 1) LLMQ_PX(kQ4_0, 1) LLMQ_PX(kQ4_1, 1) LLMQ_PX(kQ4_K, 8) LLMQ_PX(kQ5_K, 8) LLMQ_PX(kQ6_K, 8)
 LLMQ_PX(kQm4, 1) LLMQ_PX(kQm4, 2) LLMQ_PX(kQm4, 4) LLMQ_PX(kQm4, 8)
 LLMQ_PX(kQm8, 1) LLMQ_PX(kQm8, 2) LLMQ_PX(kQm8, 4) LLMQ_PX(kQm8, 8)
+LLMQ_PX(kA4, 1) LLMQ_PX(kA4, 2) LLMQ_PX(kA4, 4) LLMQ_PX(kA4, 8)
+LLMQ_PX(kA8, 1) LLMQ_PX(kA8, 2) LLMQ_PX(kA8, 4) LLMQ_PX(kA8, 8)
 #undef LLMQ_PX
 
 namespace {
@@ -30,14 +32,20 @@ bool qm_groups(const llmq_mat *w, int *seg, int *shift) {
 
 // A tile's size in 16-token and 16-row tiles, and what it measured on Q8_0
 // at 4096 x 4096 and 4096 x 11008: the time of a superblock in microseconds
-// with few workgroups, and how many of them run before that time grows.
-// (tile 0 on the K quants.)
+// with few workgroups, how many of them run before that time grows, and the
+// time before the first superblock.  (tile 0 on the K quants.)
 struct Tile {
     int tt, rt;
-    float us, full;
+    float us, full, start;
 };
-constexpr Tile kTiles[] = {{4, 16, 5.2f, 280.0f}, {4, 8, 3.6f, 328.0f}, {4, 4, 2.4f, 386.0f}, {2, 4, 1.5f, 440.0f},
-                           {1, 4, 1.2f, 510.0f},  {1, 4, 0.7f, 275.0f}, {1, 2, 0.6f, 292.0f}};
+constexpr Tile kTiles[] = {{4, 16, 5.2f, 280.0f, 4.0f}, {4, 8, 3.6f, 328.0f, 3.0f}, {4, 4, 2.4f, 386.0f, 2.0f},
+                           {2, 4, 1.5f, 440.0f, 1.0f},  {1, 4, 1.2f, 510.0f, 0.6f}, {1, 4, 0.7f, 275.0f, 0.6f},
+                           {1, 2, 0.6f, 292.0f, 0.6f}};
+
+float tile_us(const Tile &k, int64_t token_tiles, int64_t row_tiles, int64_t inputs) {
+    const float wgs = (float)((token_tiles + k.tt - 1) / k.tt * ((row_tiles + k.rt - 1) / k.rt));
+    return k.start + (float)(inputs / 256) * k.us * (wgs > k.full ? wgs / k.full : 1.0f);
+}
 
 }  // namespace
 }  // namespace planes
@@ -66,9 +74,7 @@ int gemm_planes_tile(const llmq_mat *w, int64_t T) {
     int best = -1;
     float least = 0.0f;
     for (int i = chain ? 0 : 1; i < (int)(sizeof(kTiles) / sizeof(kTiles[0])); i++) {
-        const Tile &k = kTiles[i];
-        const float wgs = (float)((tt + k.tt - 1) / k.tt * ((w->ntiles + k.rt - 1) / k.rt));
-        const float us = 4.5f + (float)(w->k / 256) * k.us * (wgs > k.full ? wgs / k.full : 1.0f);
+        const float us = 4.0f + tile_us(kTiles[i], tt, w->ntiles, w->k);
         if (best < 0 || us < least) {
             best = i;
             least = us;
@@ -145,4 +151,60 @@ int launch_gemm_planes(llmq_ctx *ctx, const llmq_mat *w, const void *rec, int64_
     case LLMQ_GGML_Q5_K: return launch_tile<kQ5_K, 8>(st, tile, a);
     default: return launch_tile<kQ6_K, 8>(st, tile, a);
     }
+}
+
+bool gemm_planes_a16_ok(const llmq_mat *w) {
+    int seg, shift;
+    return w && w->kind == MAT_QUANT && w->k % 256 == 0 && planes::qm_groups(w, &seg, &shift);
+}
+
+int launch_gemm_planes_a16(llmq_ctx *ctx, const llmq_mat *w, const uint8_t *pl, const float *sx, int64_t T, int64_t n,
+                           float *out, int64_t ldo, const float *bias, int flags) {
+    using namespace planes;
+    LLMQ_REQUIRE(gemm_planes_a16_ok(w) && n <= w->n, "gemm_planes_a16: not a matrix of this kernel");
+    Args a{};
+    a.planes = pl;
+    a.sx = sx;
+    a.codes = w->codes;
+    a.scales = reinterpret_cast<const uint8_t *>(w->scales);
+    a.zps = w->zps;
+    a.NG = (int)w->NG;
+    int seg = 8;
+    qm_groups(w, &seg, &a.gshift);
+    a.T = (int)T;
+    a.n = (int)n;
+    a.ntiles = (int)(n / 16);
+    a.NC = (int)(w->k / 32);
+    a.NSB = (int)(w->k / 256);
+    a.flags = flags;
+    a.rows_first = (T + 15) / 16 * 16 * w->k * 4 > w->ntiles * w->CK * 256;
+    a.ldo = ldo;
+    a.bias = bias ? bias : out;
+    a.out = out;
+    int tile = 1;
+    if (const char *e = getenv("LLMQ_PLANES_TILE")) {
+        tile = atoi(e) < 1 ? 1 : atoi(e) > 4 ? 4 : atoi(e);
+    } else {  // kTiles' figures hold here too: 476 x 768 x 3072 int4-ch 17.2 us with tile 2, 14.1 with 3
+        float least = 0.0f;
+        for (int i = 1; i <= 4; i++) {
+            const float us = tile_us(kTiles[i], (T + 15) / 16, a.ntiles, w->k);
+            if (i == 1 || us < least) {
+                tile = i;
+                least = us;
+            }
+        }
+    }
+    hipStream_t st = ctx->stream;
+#define LLMQ_PS(F)                                             \
+    switch (seg) {                                             \
+    case 1: return launch_tile<F, 1>(st, tile, a);             \
+    case 2: return launch_tile<F, 2>(st, tile, a);             \
+    case 4: return launch_tile<F, 4>(st, tile, a);             \
+    default: return launch_tile<F, 8>(st, tile, a);            \
+    }
+    if (w->bits == 4) {
+        LLMQ_PS(kA4)
+    }
+    LLMQ_PS(kA8)
+#undef LLMQ_PS
 }

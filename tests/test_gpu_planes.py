@@ -179,3 +179,37 @@ def test_planes_two_streams(gpu, orc):
         for o in outs[s]:
             assert torch.equal(o, ref[s])
     g.free()
+
+
+@pytest.mark.parametrize("tile", [1, 2, 3, 4])
+@pytest.mark.parametrize("fmt", [(4, 64), (4, 128), (4, 256), (4, 0), (8, 32), (8, 64), (8, 128), (8, 512), (8, 0)], ids=str)
+def test_planes_int16_activations(gpu, fmt, tile, monkeypatch):
+    """The same kernel over int16 activation codes: the int8-MFMA form's bits
+    (LLMQ_MFMA_F16=0) in every tile, with ragged tokens, the n % 32 rows
+    left to rows_i16, bias, GELU, residual and LayerNorm, and codes and
+    weights at their extremes (every partial sum then at its largest)."""
+    torch, lm, ctx = gpu
+    bits, group = fmt
+    rng = np.random.default_rng(bits + group)
+    for t, n, k, big in ((2, 64, 512, True), (17, 70, 512, False), (65, 300, 1024, False), (130, 96, 1536, True)):
+        w = rng.normal(0, 0.05, (k, n)).astype(np.float32)
+        x = rng.normal(0, 1, (t, k)).astype(np.float32)
+        if big:  # codes near +-32767 against u - zp at its ends
+            w = np.where(rng.random((k, n)) < 0.97, 0.1, -1e-4).astype(np.float32)
+            x = (rng.uniform(0.999, 1.0, (t, k)) * np.where(np.arange(t)[:, None] % 2, -1, 1)).astype(np.float32)
+        g = lm.HipQuantMatrix.from_f32(ctx, w, bits, group, False, True)
+        b, res = dev(torch, rng.normal(0, 1, n).astype(np.float32)), rng.normal(0, 1, (t, n)).astype(np.float32)
+        ln = (dev(torch, rng.uniform(0.5, 1.5, k).astype(np.float32)), dev(torch, rng.normal(0, 0.1, k).astype(np.float32)))
+        got = []
+        for env in ({"LLMQ_MFMA_F16": "0"}, {"LLMQ_MFMA_F16": "1", "LLMQ_PLANES_TILE": str(tile)}):
+            for name, v in env.items():
+                monkeypatch.setenv(name, v)
+            for opt in ({"gelu": True}, {"resid": True}, {} if big else {"ln": ln}):
+                print("planes a16", fmt, tile, t, n, k, env, opt.keys(), flush=True)
+                out = dev(torch, res)
+                lm.linear(ctx, out, dev(torch, x), g, b, **opt)
+                torch.cuda.synchronize()
+                got.append(out.cpu().numpy().view(np.uint32))
+        for i in range(3):
+            assert np.array_equal(got[i], got[3 + i]), (t, n, k, i)
+        g.free()

@@ -64,6 +64,44 @@ def test_ikv_store_and_attend_bit_exact(gpu, orc, T, pos0, MT, NH, HS, spread):
     assert len(bad) == 0, (len(bad), bad[:4].tolist(), got[tuple(bad[0])], want[tuple(bad[0])])
 
 
+PROMPT_EDGES = [
+    # (T, pos0, n_head, head_dim, scale of the values); more than 256 (token, head) pairs, 512 at
+    # head_dim 128, take the prompt kernel
+    (2, 0, 129, 64, 1.0), (15, 49, 18, 64, 1.0), (16, 48, 17, 64, 1.0), (17, 48, 16, 64, 1.0),  # tiles, runs
+    (33, 479, 8, 64, 1.0), (33, 480, 8, 64, 1.0), (20, 1004, 13, 64, 1.0), (20, 1005, 13, 64, 1.0),  # runs a wave
+    (40, 2008, 7, 64, 1.0), (40, 2009, 7, 64, 1.0),  # the longest context, and past it
+    (16, 48, 16, 64, 1.0), (9, 120, 57, 128, 1.0), (65, 448, 8, 128, 1.0), (30, 1700, 18, 128, 1.0),
+    (19, 250, 14, 64, 0.0), (19, 250, 14, 64, 9000.0),  # equal scales; scales past int32
+]
+
+
+@pytest.mark.parametrize("T,pos0,NH,HS,vscale", PROMPT_EDGES)
+def test_ikv_prompt_edges_bit_exact(gpu, orc, T, pos0, NH, HS, vscale):
+    """Several tokens at the edges of the prompt kernel's tiles, runs and
+    register sets: outputs bit-identical to the oracle."""
+    torch, lm, ctx = gpu
+    C, n, MT = NH * HS, pos0 + T, 2064
+    rng = np.random.default_rng(7 * T + pos0 + HS)
+    qkv = rng.normal(0, 1, (n, 3 * C)).astype(np.float32)
+    qkv[:, :C] *= np.exp(rng.normal(0, 2, (n, 1))).astype(np.float32)  # flat and peaked attention
+    qkv[:, 2 * C:] *= np.float32(vscale)
+    qkv[n - 1, :HS] = 0.0  # an all-zero query: equal weights
+    qkv[n - 2, :HS] = np.where(np.arange(HS) % 2, 3.0, -3.0)  # both ends of int16
+    note("ikv prompt", T, pos0, NH, HS, vscale)
+    kv, okv = lm.IntAttnKV(ctx, 1, MT, NH, HS), orc.IntAttnKV(1, MT, NH, HS)
+    kv.store(0, 0, dev(torch, qkv))
+    for p in range(n):
+        okv.store(0, p, qkv[p, C:2 * C], qkv[p, 2 * C:])
+    if vscale == 9000.0:
+        assert (okv.vq[0] < 0).any()
+    out = torch.zeros((T, C), dtype=torch.float32, device="cuda")
+    kv.attend(out, dev(torch, qkv[pos0:]), 0, pos0)
+    torch.cuda.synchronize()
+    want, got = okv.attend(qkv[pos0:], 0, T, pos0), out.cpu().numpy()
+    bad = np.argwhere(got.view(np.uint32) != want.view(np.uint32))
+    assert len(bad) == 0, (len(bad), bad[:4].tolist(), got[tuple(bad[0])], want[tuple(bad[0])])
+
+
 def test_ikv_shape_checks(gpu):
     torch, lm, ctx = gpu
     with pytest.raises(lm.LlmqError, match="max_t % 16"):

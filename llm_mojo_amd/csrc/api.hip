@@ -47,7 +47,46 @@ int llmq_set_error(int code, const char *fmt, ...) {
 }
 
 
+namespace {
+
+bool capturing(hipStream_t s) {
+    hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
+    const bool known = hipStreamIsCapturing(s, &c) == hipSuccess;
+    if (!known) (void)hipGetLastError();
+    return known && c != hipStreamCaptureStatusNone;
+}
+
+// Puts ws_event behind the workspaces' uses on the stream that used them
+// last, if it is not there yet.  Nothing is recorded into a capture.
+bool ws_record(llmq_ctx *ctx) {
+    if (ctx->ws_recorded) return true;
+    if (capturing(ctx->ws_stream)) return false;
+    ctx->ws_recorded = (ctx->ws_event || hipEventCreateWithFlags(&ctx->ws_event, hipEventDisableTiming) == hipSuccess) &&
+                       hipEventRecord(ctx->ws_event, ctx->ws_stream) == hipSuccess;
+    if (!ctx->ws_recorded) (void)hipGetLastError();
+    return ctx->ws_recorded;
+}
+
+// The context's stream takes a workspace over: it waits for the stream that
+// used one last, whichever streams the context was given in between, and
+// with that for every use before (also where the handle is the same again:
+// the stream may be a new one at an old one's address).  While the context's
+// stream is being captured it uses nothing yet, and nothing changes here; a
+// stream left while it was being captured is waited for from the capture's
+// end on.
+int ws_take(llmq_ctx *ctx) {
+    if (capturing(ctx->stream)) return LLMQ_OK;
+    if (ctx->ws_stream && (ctx->ws_stream != ctx->stream || ctx->ws_recorded) && ws_record(ctx))
+        LLMQ_HIP(hipStreamWaitEvent(ctx->stream, ctx->ws_event, 0));
+    ctx->ws_stream = ctx->stream;
+    ctx->ws_recorded = false;
+    return LLMQ_OK;
+}
+
+}  // namespace
+
 int ctx_workspace(llmq_ctx *ctx, size_t bytes, void **p, int slot) {
+    RC(ws_take(ctx));
     if (bytes > ctx->ws_bytes[slot]) {
         LLMQ_HIP(hipStreamSynchronize(ctx->stream));
         if (ctx->ws[slot]) hipFree(ctx->ws[slot]);
@@ -59,7 +98,6 @@ int ctx_workspace(llmq_ctx *ctx, size_t bytes, void **p, int slot) {
         ctx->ws_bytes[slot] = want;
     }
     *p = ctx->ws[slot];
-    ctx->ws_used = true;
     return LLMQ_OK;
 }
 
@@ -110,18 +148,8 @@ int llmq_destroy(llmq_ctx *ctx) {
 int llmq_set_stream(llmq_ctx *ctx, void *s) {
     LLMQ_REQUIRE(ctx, "set_stream: null context");
     const hipStream_t to = s ? (hipStream_t)s : ctx->own_stream;
-    if (to != ctx->stream && ctx->ws_used) {
-        // the workspaces are shared by every stream the context is given: work on the new one waits
-        // for what is still reading them on the old one (not within a capture, which cannot wait on it)
-        hipStreamCaptureStatus a = hipStreamCaptureStatusNone, b = a;
-        if (hipStreamIsCapturing(ctx->stream, &a) == hipSuccess && hipStreamIsCapturing(to, &b) == hipSuccess &&
-            a == hipStreamCaptureStatusNone && b == hipStreamCaptureStatusNone &&
-            (ctx->ws_event || hipEventCreateWithFlags(&ctx->ws_event, hipEventDisableTiming) == hipSuccess) &&
-            hipEventRecord(ctx->ws_event, ctx->stream) == hipSuccess)
-            (void)hipStreamWaitEvent(to, ctx->ws_event, 0);
-        (void)hipGetLastError();
-        ctx->ws_used = false;
-    }
+    // the event goes behind the workspaces' uses now, while the stream that is left surely exists
+    if (to != ctx->stream && ctx->ws_stream == ctx->stream) (void)ws_record(ctx);
     ctx->stream = to;
     return LLMQ_OK;
 }

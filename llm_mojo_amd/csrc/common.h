@@ -39,8 +39,9 @@ struct llmq_ctx {
     // several-token float-activation matmul
     void *ws[2] = {nullptr, nullptr};
     size_t ws_bytes[2] = {0, 0};
-    bool ws_used = false;           // handed out since the last change of stream
-    hipEvent_t ws_event = nullptr;  // llmq_set_stream orders the new stream after the workspaces' users
+    hipStream_t ws_stream = nullptr;  // the stream that used a workspace last
+    hipEvent_t ws_event = nullptr;    // behind its uses there, once
+    bool ws_recorded = false;         // this is true
     void *scratch = nullptr;  // this device's no-allocation scratch (llmq_linear_noalloc), from llmq_init
 };
 

@@ -169,25 +169,27 @@ LLMQ_API int llmq_quantize_rows(llmq_ctx *ctx, const float *x, int64_t T, int64_
  * run in integers (matmul_rows_a16, 419-509); for a GGUF matrix or a
  * QuantMatrix with a16 = 0 the float path (matmul_rows, 285-349, over
  * GGUFMatrix.dot_row / QuantMatrix.dot_row, tensor.mojo:431-482).
- * flags: LLMQ_BIAS | LLMQ_GELU | LLMQ_RESID. */
+ * flags: LLMQ_BIAS | LLMQ_GELU | LLMQ_RESID.  The float path's sums are in
+ * float32 in an order that depends on the shape and on T: a token's last
+ * bits may differ between calls of different T, not with its neighbours. */
 LLMQ_API int llmq_linear(llmq_ctx *ctx, float *out, const float *x, const llmq_mat *w, const float *bias, int64_t T,
                          int64_t IN, int64_t OUT, int flags);
 /* No counterpart in the reference: llmq_linear for callers that cannot
  * allocate device memory (code under HIP graph capture, serving loops,
  * harnesses that forbid hipMalloc).  Same arguments, kernels and results
  * (bit for bit) as llmq_linear; where llmq_linear grows the context's
- * workspace (the a16 prompt GEMM's int16 activation codes and row scales,
- * the Q4_K matmul's fp16 activation record), this form uses a fixed
+ * workspace (the a16 prompt GEMM's int16 activation codes, row scales and
+ * fp16 planes, the Q4_K matmul's fp16 activation record), this form uses a fixed
  * per-GPU scratch array of LLMQ_NOALLOC_SCRATCH_BYTES that each GPU the
  * library runs on holds until the process ends.  It calls no hipMalloc /
  * hipFree.  Sizes needing more scratch than that (a16: T x IN x 2 bytes
  * and T x 4, each rounded up to 256; Q4_K: the record's ~4.4 x T x IN
- * bytes, T rounded up to 16) return LLMQ_EINVAL; other float-activation
- * formats take as many tokens at a time as the scratch holds.  An a16 matrix
+ * bytes, T rounded up to 16) return LLMQ_EINVAL; the other formats use no
+ * scratch.  An a16 matrix
  * in groups of 32, or of whole 256-input superblocks, also puts its prompt
  * GEMM's fp16 activation planes there (T x IN x 4 bytes, T rounded up to 16)
  * when they fit, else runs the int8-MFMA form of the GEMM (the same bits).
- * Every call on one GPU shares the array: calls that overlap in time on one
+ * Every call that uses it shares the array: calls that overlap in time on one
  * GPU (different streams or threads) race; calls ordered on one stream do
  * not.  Nothing in the scratch needs to start at zero (each call writes all
  * it reads). */

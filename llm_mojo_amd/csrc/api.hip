@@ -529,13 +529,13 @@ int llmq_linear_noalloc(llmq_ctx *ctx, float *out, const float *x, const llmq_ma
     LLMQ_REQUIRE(T >= 1, "linear_noalloc: T must be >= 1");
     if (is_float_act(w)) {
         // the one-token GEMV uses no scratch; several tokens of Q4_K keep
-        // their fp16 activation record there (the other types use none)
+        // their fp16 activation record there (the other types use no memory)
         if (T == 1) return launch_gguf_gemv(ctx, w, x, out, bias, flags, nullptr, 0);
         return launch_gguf_gemm(ctx, w, x, IN, T, out, OUT, bias, flags, ctx->scratch, LLMQ_NOALLOC_SCRATCH_BYTES);
     }
     // the least the prompt GEMM keeps there: T x IN int16 codes and T float
-    // scales, each rounded up to 256 bytes (their fp16
-    // planes go there too when they fit, else take the int8-MFMA form)
+    // scales, each rounded up to 256 bytes (their fp16 planes, where the
+    // matrix takes that form, go there too when they fit)
     const int64_t need = ((T * IN * 2 + 255) & ~(int64_t)255) + ((T * 4 + 255) & ~(int64_t)255);
     LLMQ_REQUIRE(need <= (int64_t)LLMQ_NOALLOC_SCRATCH_BYTES,
                  "linear_noalloc: %lld tokens x %lld inputs need %lld bytes of scratch, the maximum is %d",

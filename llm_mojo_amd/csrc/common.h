@@ -385,15 +385,13 @@ inline int float_act_type(const llmq_mat *w) {
 // log2 of the chunks per group of a QuantMatrix (31 for per-channel: every
 // chunk of a row is group 0); groups are powers of two times 32 otherwise.
 int qm_cpg_shift(const llmq_mat *w);
-// Several-token GGUF matmul.  Matrices of whole superblocks take the fp16
-// matrix cores over an h16 record of x (gguf_gemm16.hip for a few tokens of
-// Q4_K, gemm_planes.hip): `rec` of `rec_cap` bytes when given, the context's
-// workspace slot 1 when rec_cap < 0, and the fp32 matrix cores
-// (gguf_gemm.hip) when rec_cap == 0; LLMQ_GEMM_H16=0 forces those.  Types
-// other than Q4_K need no record to be accepted: without room for one, and
-// under graph capture over the context's workspace (which a later call may
-// move), they take as many tokens at a time as there is room for, or the
-// fp32 kernel.
+// Several-token GGUF matmul.  Q4_K matrices of whole superblocks take the
+// fp16 matrix cores over an h16 record of x (gguf_gemm16.hip for a few
+// tokens, gemm_planes.hip): `rec` of `rec_cap` bytes when given, the
+// context's workspace slot 1 when rec_cap < 0, and the fp32 matrix cores
+// (gguf_gemm.hip) when rec_cap == 0.  The other types need no memory: the
+// bf16 matrix cores over x itself (gemm_planes.hip) or the fp32 ones.
+// LLMQ_GEMM_H16=0 forces the fp32 matrix cores.
 int launch_gguf_gemm(llmq_ctx *ctx, const llmq_mat *w, const float *x, int64_t ldx, int64_t T, float *out,
                      int64_t ldo, const float *bias, int flags, void *rec = nullptr, int64_t rec_cap = -1);
 // The h16 record (gguf_gemm16.hip): its size for T tokens of K inputs, the
@@ -401,16 +399,17 @@ int launch_gguf_gemm(llmq_ctx *ctx, const llmq_mat *w, const float *x, int64_t l
 int64_t h16_rec_bytes(int64_t T, int64_t K);
 void h16_rec_parts(void *rec, int64_t T, int64_t K, uint8_t **planes, _Float16 **sums, float **inv);
 bool gguf_gemm_h16_ok(const llmq_mat *w);
-// The matmul over that record for prompts and the other float-activation
-// formats (gemm_planes.hip): any GGUF or A16 = False matrix of whole
-// superblocks whose groups are a power of two times 32 or the row.
-// gemm_planes_tile is the tile for T tokens, or -1 where the fp32 kernel is
-// the faster one; an output's bits depend on the tile and its own token only.
+// The matmul of prompts (gemm_planes.hip): Q4_K over that record, any other
+// GGUF or A16 = False matrix of whole superblocks, whose groups are a power of
+// two times 32 or the row, over x itself.  gemm_floats_tile is the tile for T
+// tokens, or -1 where the fp32 kernel is the faster one; an output's bits
+// depend on the tile and its own token only.
 bool gemm_planes_ok(const llmq_mat *w);
-int gemm_planes_tile(const llmq_mat *w, int64_t T);
+int gemm_floats_tile(const llmq_mat *w, int64_t T);
 int launch_gemm_planes(llmq_ctx *ctx, const llmq_mat *w, const void *rec, int64_t T, float *out, int64_t ldo,
-                       const float *bias, int flags, int tile);
-// (rows: a wave a superblock of a token, for one token tile of Q4_K)
+                       const float *bias, int flags);
+int launch_gemm_floats(llmq_ctx *ctx, const llmq_mat *w, const float *x, int64_t ldx, int64_t T, float *out,
+                       int64_t ldo, const float *bias, int flags, int tile);
 // The same kernel over int16 activation codes as fp16 planes (gemm_mfma.hip's
 // layout; sx the tokens' scales): the first n rows of w, whose K is whole
 // superblocks and whose groups are a power of two times 32 or the row; the
@@ -418,6 +417,8 @@ int launch_gemm_planes(llmq_ctx *ctx, const llmq_mat *w, const void *rec, int64_
 bool gemm_planes_a16_ok(const llmq_mat *w);
 int launch_gemm_planes_a16(llmq_ctx *ctx, const llmq_mat *w, const uint8_t *pl, const float *sx, int64_t T, int64_t n,
                            float *out, int64_t ldo, const float *bias, int flags);
+// rows: a wave a superblock of a token (one token tile), else a workgroup a
+// superblock of 16 tokens
 int launch_act_h16(llmq_ctx *ctx, const float *x, int64_t ldx, int64_t T, int64_t K, void *rec, bool rows = false);
 // The batch-decode chain's forms of that matmul (gguf_gemm16.hip): the
 // input may be an "h16s" record (a scale per 16 inputs of a token, written

@@ -5,9 +5,8 @@
 namespace planes {
 
 #define LLMQ_PX(F, SEG) extern template int launch_tile<F, SEG>(hipStream_t, int, const Args &);
-LLMQ_PX(kQ8_0, 1) LLMQ_PX(kQ4_0, 1) LLMQ_PX(kQ4_1, 1) LLMQ_PX(kQ4_K, 8) LLMQ_PX(kQ5_K, 8) LLMQ_PX(kQ6_K, 8)
-LLMQ_PX(kQm4, 1) LLMQ_PX(kQm4, 2) LLMQ_PX(kQm4, 4) LLMQ_PX(kQm4, 8)
-LLMQ_PX(kQm8, 1) LLMQ_PX(kQm8, 2) LLMQ_PX(kQm8, 4) LLMQ_PX(kQm8, 8)
+LLMQ_PX(kQ8_0, 1) LLMQ_PX(kQ4_0, 1) LLMQ_PX(kQ4_1, 1) LLMQ_PX(kQ4_K, 8) LLMQ_PX(kQ5_K, 1) LLMQ_PX(kQ6_K, 8)
+LLMQ_PX(kQm4, 1) LLMQ_PX(kQm4, 8) LLMQ_PX(kQm8, 1) LLMQ_PX(kQm8, 8)
 LLMQ_PX(kA4, 1) LLMQ_PX(kA4, 2) LLMQ_PX(kA4, 4) LLMQ_PX(kA4, 8)
 LLMQ_PX(kA8, 1) LLMQ_PX(kA8, 2) LLMQ_PX(kA8, 4) LLMQ_PX(kA8, 8)
 #undef LLMQ_PX
@@ -56,45 +55,118 @@ bool gemm_planes_ok(const llmq_mat *w) {
     return w->kind == MAT_GGUF || planes::qm_groups(w, &seg, &shift);
 }
 
-// The tile with the least time by kTiles' figures; -1 where the fp32 kernel
-// is faster: it reads x itself, without the record's 4.5 us, at 22 MAC a
-// picosecond (16 tokens of 4096 x 4096: 12.3 us against 14, 64 tokens 50 against 18).
-// Q4_K has a kernel of its own for few tokens.
-int gemm_planes_tile(const llmq_mat *w, int64_t T) {
+// LLMQ_PLANES_TILE, or -1.
+static int forced_tile() {
+    const char *e = getenv("LLMQ_PLANES_TILE");
+    if (!e) return -1;
+    const int t = atoi(e);
+    return t < 0 ? 0 : t > 6 ? 6 : t;
+}
+
+// Q4_K's tile, the one with the least time by kTiles' figures (few tokens
+// have a kernel of their own).
+static int q4k_tile(const llmq_mat *w, int64_t T) {
     using namespace planes;
-    if (const char *e = getenv("LLMQ_PLANES_TILE")) {
-        const int t = atoi(e);
-        return t < 0 ? 0 : t > 6 ? 6 : t;
-    }
-    const int64_t tt = (T + 15) / 16;
-    int seg = 8, shift;
-    if (w->kind == MAT_QUANT) qm_groups(w, &seg, &shift);
-    const int ty = float_act_type(w);
-    const bool chain = seg == 8 && ty != LLMQ_GGML_Q8_0 && ty != LLMQ_GGML_Q4_0 && ty != LLMQ_GGML_Q4_1;
-    int best = -1;
+    int best = forced_tile();
+    if (best >= 0) return best;
     float least = 0.0f;
-    for (int i = chain ? 0 : 1; i < (int)(sizeof(kTiles) / sizeof(kTiles[0])); i++) {
-        const float us = 4.0f + tile_us(kTiles[i], tt, w->ntiles, w->k);
+    for (int i = 0; i < (int)(sizeof(kTiles) / sizeof(kTiles[0])); i++) {
+        const float us = tile_us(kTiles[i], (T + 15) / 16, w->ntiles, w->k);
         if (best < 0 || us < least) {
             best = i;
             least = us;
         }
     }
-    const float fp32_us = 3.5f + (float)T * (float)w->k * (float)w->n / 22e6f;
-    return ty != LLMQ_GGML_Q4_K && fp32_us < least ? -1 : best;
+    return best;
 }
 
-int launch_gemm_planes(llmq_ctx *ctx, const llmq_mat *w, const void *rec, int64_t T, float *out, int64_t ldo,
-                       const float *bias, int flags, int tile) {
+// The tiles over floats: what a superblock costs in microseconds with one
+// workgroup on the fullest of the 256 CUs, and each further one there; 4 us
+// before the first.  Fitted to 237 calls of Q8_0, int4-g32 and int8-ch (16
+// to 1024 tokens, 768 to 8192 inputs, 768 to 12000 rows), 6 to 12 % off a
+// tile's times.  The fp32 kernel does 22 MAC a picosecond (16 tokens of 4096
+// x 4096: 13 us against 16; 64 tokens 50 against 18).  With these the choice
+// is within 1 % of the best of the six on all of those calls, and within 9 %
+// on 79 of Q6_K, whose products are twice as many.
+int gemm_floats_tile(const llmq_mat *w, int64_t T) {
     using namespace planes;
-    LLMQ_REQUIRE(gemm_planes_ok(w) && tile >= 0, "gemm_planes: not a matrix of this kernel");
-    LLMQ_REQUIRE(rec && out && T > 0, "gemm_planes: bad arguments");
+    struct FloatTile {
+        int tt, rt;
+        float us, more;
+    };
+    static constexpr FloatTile tiles[] = {{2, 16, 4.10f, 3.33f}, {2, 8, 2.53f, 3.17f}, {1, 8, 1.60f, 2.06f},
+                                          {1, 4, 1.02f, 1.28f},  {1, 2, 0.73f, 0.69f}};
+    int best = forced_tile();
+    if (best >= 0) return best;
+    float least = 2.5f + (float)T * (float)w->k * (float)w->n / 22e6f;
+    for (int i = 0; i < (int)(sizeof(tiles) / sizeof(tiles[0])); i++) {
+        const FloatTile &k = tiles[i];
+        const int64_t wgs = ((T + 15) / 16 + k.tt - 1) / k.tt * ((w->ntiles + k.rt - 1) / k.rt);
+        const float us = 4.0f + (float)(w->k / 256) * (k.us + k.more * (float)((wgs + 255) / 256 - 1));
+        if (us < least) {
+            best = i;
+            least = us;
+        }
+    }
+    return best;
+}
+
+namespace planes {
+namespace {
+
+// The weights' and the outputs' side of a call (seg: chunks that share a scale).
+int args(const llmq_mat *w, int64_t T, float *out, int64_t ldo, const float *bias, int flags, Args *a, int *seg) {
+    LLMQ_REQUIRE(gemm_planes_ok(w), "gemm_planes: not a matrix of this kernel");
+    LLMQ_REQUIRE(out && T > 0, "gemm_planes: bad arguments");
     LLMQ_REQUIRE(!(flags & LLMQ_BIAS) || bias, "gemm_planes: LLMQ_BIAS without a bias");
-    const int64_t T16 = (T + 15) / 16 * 16, NSB = w->k / 256;
-    const int64_t ntc = (w->ntiles * w->CK + LLMQ_PAD_CHUNKS) * 16, nts = (w->ntiles * w->NG + LLMQ_PAD_CHUNKS) * 16;
-    LLMQ_REQUIRE(ntc * 16 < (int64_t)kLlmqOOB && h16_rec_bytes(T, w->k) < (int64_t)kLlmqOOB,
-                 "gemm_planes: operands too large");
-    Args a{};
+    const int64_t T16 = (T + 15) / 16 * 16;
+    const int64_t ntc = (w->ntiles * w->CK + LLMQ_PAD_CHUNKS) * 16;
+    LLMQ_REQUIRE(ntc * 16 < (int64_t)kLlmqOOB, "gemm_planes: operands too large");
+    *a = Args{};
+    a->codes = w->codes;
+    *seg = 8;
+    if (w->kind == MAT_QUANT) {
+        qm_groups(w, seg, &a->gshift);
+        a->scales = reinterpret_cast<const uint8_t *>(w->scales);
+        a->zps = w->zps;
+        a->NG = (int)w->NG;
+    } else if (w->ggml_type == LLMQ_GGML_Q4_1) {
+        a->scales = reinterpret_cast<const uint8_t *>(w->g_meta32);
+    } else if (w->ggml_type == LLMQ_GGML_Q8_0 || w->ggml_type == LLMQ_GGML_Q4_0) {
+        a->scales = reinterpret_cast<const uint8_t *>(w->g_meta16);
+    } else {
+        a->sb = reinterpret_cast<const uint8_t *>(w->g_sb16);
+        if (w->ggml_type == LLMQ_GGML_Q5_K) {
+            a->bits = reinterpret_cast<const uint8_t *>(w->g_bits32);
+        } else if (w->ggml_type == LLMQ_GGML_Q6_K) {
+            a->bits = reinterpret_cast<const uint8_t *>(w->g_bits64);
+            a->sbd = reinterpret_cast<const uint8_t *>(w->g_meta16);
+        }
+    }
+    a->T = (int)T;
+    a->n = (int)w->n;
+    a->ntiles = (int)w->ntiles;
+    a->NC = (int)(w->k / 32);
+    a->NSB = (int)(w->k / 256);
+    a->flags = flags;
+    a->rows_first = T16 * w->k * 4 > ntc * 16;
+    a->ldo = ldo;
+    a->bias = bias ? bias : out;
+    a->out = out;
+    return LLMQ_OK;
+}
+
+}  // namespace
+}  // namespace planes
+
+int launch_gemm_planes(llmq_ctx *ctx, const llmq_mat *w, const void *rec, int64_t T, float *out, int64_t ldo,
+                       const float *bias, int flags) {
+    using namespace planes;
+    Args a;
+    int seg;
+    RC(args(w, T, out, ldo, bias, flags, &a, &seg));
+    LLMQ_REQUIRE(gguf_gemm_h16_ok(w) && rec && h16_rec_bytes(T, w->k) < (int64_t)kLlmqOOB,
+                 "gemm_planes: not a record of this kernel");
     uint8_t *pl;
     _Float16 *su;
     float *iv;
@@ -102,54 +174,28 @@ int launch_gemm_planes(llmq_ctx *ctx, const llmq_mat *w, const void *rec, int64_
     a.planes = pl;
     a.sums = reinterpret_cast<const uint8_t *>(su);
     a.inv = reinterpret_cast<const uint8_t *>(iv);
-    a.codes = w->codes;
-    int seg = 8;
-    if (w->kind == MAT_QUANT) {
-        qm_groups(w, &seg, &a.gshift);
-        a.scales = reinterpret_cast<const uint8_t *>(w->scales);
-        a.zps = w->zps;
-        a.NG = (int)w->NG;
-    } else if (w->ggml_type == LLMQ_GGML_Q4_1) {
-        a.scales = reinterpret_cast<const uint8_t *>(w->g_meta32);
-    } else if (w->ggml_type == LLMQ_GGML_Q8_0 || w->ggml_type == LLMQ_GGML_Q4_0) {
-        a.scales = reinterpret_cast<const uint8_t *>(w->g_meta16);
-    } else {
-        a.sb = reinterpret_cast<const uint8_t *>(w->g_sb16);
-        if (w->ggml_type == LLMQ_GGML_Q5_K) {
-            a.bits = reinterpret_cast<const uint8_t *>(w->g_bits32);
-        } else if (w->ggml_type == LLMQ_GGML_Q6_K) {
-            a.bits = reinterpret_cast<const uint8_t *>(w->g_bits64);
-            a.sbd = reinterpret_cast<const uint8_t *>(w->g_meta16);
-        }
-    }
-    a.T = (int)T;
-    a.n = (int)w->n;
-    a.ntiles = (int)w->ntiles;
-    a.NC = (int)(w->k / 32);
-    a.NSB = (int)NSB;
-    a.flags = flags;
-    a.rows_first = T16 * w->k * 4 > ntc * 16;
-    a.ldo = ldo;
-    a.bias = bias ? bias : out;
-    a.out = out;
+    return launch_tile<kQ4_K, 8>(ctx->stream, q4k_tile(w, T), a);
+}
+
+int launch_gemm_floats(llmq_ctx *ctx, const llmq_mat *w, const float *x, int64_t ldx, int64_t T, float *out,
+                       int64_t ldo, const float *bias, int flags, int tile) {
+    using namespace planes;
+    Args a;
+    int seg;
+    RC(args(w, T, out, ldo, bias, flags, &a, &seg));
+    LLMQ_REQUIRE(tile >= 0 && x && ldx >= w->k && T * ldx * 4 < (int64_t)kLlmqOOB, "gemm_floats: bad arguments");
+    a.x = x;
+    a.ldx = ldx;
     hipStream_t st = ctx->stream;
-    switch (float_act_type(w)) {
-#define LLMQ_PS(F)                                             \
-    switch (seg) {                                             \
-    case 1: return launch_tile<F, 1>(st, tile, a);             \
-    case 2: return launch_tile<F, 2>(st, tile, a);             \
-    case 4: return launch_tile<F, 4>(st, tile, a);             \
-    default: return launch_tile<F, 8>(st, tile, a);            \
-    }
-    case kQmFloat4: LLMQ_PS(kQm4)
-    case kQmFloat8: LLMQ_PS(kQm8)
-#undef LLMQ_PS
+    switch (float_act_type(w)) {  // (groups of 64 and 128 take their scale a chunk at a time)
+    case kQmFloat4: return seg == 8 ? launch_tile<kQm4, 8>(st, tile, a) : launch_tile<kQm4, 1>(st, tile, a);
+    case kQmFloat8: return seg == 8 ? launch_tile<kQm8, 8>(st, tile, a) : launch_tile<kQm8, 1>(st, tile, a);
     case LLMQ_GGML_Q8_0: return launch_tile<kQ8_0, 1>(st, tile, a);
     case LLMQ_GGML_Q4_0: return launch_tile<kQ4_0, 1>(st, tile, a);
     case LLMQ_GGML_Q4_1: return launch_tile<kQ4_1, 1>(st, tile, a);
-    case LLMQ_GGML_Q4_K: return launch_tile<kQ4_K, 8>(st, tile, a);
-    case LLMQ_GGML_Q5_K: return launch_tile<kQ5_K, 8>(st, tile, a);
-    default: return launch_tile<kQ6_K, 8>(st, tile, a);
+    case LLMQ_GGML_Q5_K: return launch_tile<kQ5_K, 1>(st, tile, a);
+    case LLMQ_GGML_Q6_K: return launch_tile<kQ6_K, 8>(st, tile, a);
+    default: return llmq_set_error(LLMQ_EUNSUPPORTED, "gemm_floats: type %d", float_act_type(w));
     }
 }
 

@@ -4,8 +4,6 @@
 namespace planes {
 
 template int launch_tile<kQm4, 1>(hipStream_t, int, const Args &);
-template int launch_tile<kQm4, 2>(hipStream_t, int, const Args &);
-template int launch_tile<kQm4, 4>(hipStream_t, int, const Args &);
 template int launch_tile<kQm4, 8>(hipStream_t, int, const Args &);
 
 }  // namespace planes

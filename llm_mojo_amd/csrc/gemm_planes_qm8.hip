@@ -4,8 +4,6 @@
 namespace planes {
 
 template int launch_tile<kQm8, 1>(hipStream_t, int, const Args &);
-template int launch_tile<kQm8, 2>(hipStream_t, int, const Args &);
-template int launch_tile<kQm8, 4>(hipStream_t, int, const Args &);
 template int launch_tile<kQm8, 8>(hipStream_t, int, const Args &);
 
 }  // namespace planes

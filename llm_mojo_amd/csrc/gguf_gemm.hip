@@ -1,6 +1,6 @@
-// Several-token GGUF matmul where the fp16 matrix cores (gguf_gemm16.hip,
-// gemm_planes.hip) are not the faster form or not to be had: matmul_rows for T > 1 over a GGUFMatrix
-// (kernels.mojo:314-349: rows dequantized, gguf.mojo:178-297, then a float
+// Several-token GGUF matmul where the 16-bit matrix cores (gguf_gemm16.hip,
+// gemm_planes.hip) are not the faster form or do not take the matrix:
+// matmul_rows for T > 1 over a GGUFMatrix (kernels.mojo:314-349: rows dequantized, gguf.mojo:178-297, then a float
 // tile matmul, with store_out's bias / GELU / residual), on the fp32 matrix
 // cores (v_mfma_f32_16x16x4f32).
 //
@@ -15,14 +15,11 @@
 // weights and loads its token's 64 activations into registers, and MFMA
 // step t multiplies input 64 (l / 16) + t of both.  The waves' 16 x 16
 // partial sums are added in LDS in wave order.
-#include <algorithm>
-
 #include "common.h"
 
 namespace {
 
 constexpr uint32_t kOOB = 0x80000000u;
-constexpr int64_t kMaxRec = 1 << 30;  // bytes of workspace for an activation record; longer prompts go in parts
 
 typedef float v4f __attribute__((ext_vector_type(4)));
 
@@ -234,23 +231,9 @@ int launch_gguf_gemm(llmq_ctx *ctx, const llmq_mat *w, const float *x, int64_t l
     const int64_t nts = (w->ntiles * w->NG + LLMQ_PAD_CHUNKS) * 16;
     LLMQ_REQUIRE(ntc * 16 < (int64_t)kOOB && T * ldx * 4 < (int64_t)kOOB, "gguf_gemm: operands too large");
     LLMQ_REQUIRE(T <= 16 * 65535LL, "gguf_gemm: too many tokens");
-    const int tile = rec_cap != 0 && gemm_planes_ok(w) && !(he && he[0] == '0') ? gemm_planes_tile(w, T) : -1;
-    if (tile >= 0) {
-        const int64_t need = h16_rec_bytes(T, w->k), tok16 = h16_rec_bytes(16, w->k);
-        int64_t cap = rec_cap;
-        if (rec_cap < 0) {
-            hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-            if (hipStreamIsCapturing(ctx->stream, &cs) != hipSuccess) (void)hipGetLastError();
-            cap = std::max(tok16, std::min<int64_t>(need, kMaxRec / tok16 * tok16));
-            if (cs != hipStreamCaptureStatusNone || ctx_workspace(ctx, (size_t)cap, &rec, 1) != LLMQ_OK) cap = 0;
-        }
-        const int64_t step = need <= cap ? T : cap / tok16 * 16;
-        for (int64_t t = 0; step > 0 && t < T; t += step) {
-            const int64_t n = std::min(step, T - t);
-            RC(launch_act_h16(ctx, x + t * ldx, ldx, n, w->k, rec));
-            RC(launch_gemm_planes(ctx, w, rec, n, out + t * ldo, ldo, bias, flags, tile));
-        }
-        if (step > 0) return LLMQ_OK;
+    if (!gguf_gemm_h16_ok(w) && gemm_planes_ok(w) && !(he && he[0] == '0')) {
+        const int tile = gemm_floats_tile(w, T);
+        if (tile >= 0) return launch_gemm_floats(ctx, w, x, ldx, T, out, ldo, bias, flags, tile);
     }
     GArgs a{};
     const int t = float_act_type(w);

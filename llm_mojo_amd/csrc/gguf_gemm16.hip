@@ -594,7 +594,7 @@ int launch_gguf_gemm_h16(llmq_ctx *ctx, const llmq_mat *w, const void *rec, int6
                  "gguf_gemm_h16: operands too large");
     // prompts: 48 tokens of 2048 x 5632 measured 15.4 us here and 14.5 there, 100 of 4096 x 4096 49 and 25
     if (!fused && T16 / 16 >= kPT)
-        return launch_gemm_planes(ctx, w, rec, T, out, ldo, bias, flags, gemm_planes_tile(w, T));
+        return launch_gemm_planes(ctx, w, rec, T, out, ldo, bias, flags);
     HArgs a{};
     a.codes = w->codes;
     a.codes_bytes = (uint32_t)(ntc * 16);

@@ -4,7 +4,8 @@ rows that fill none, one and a part of them; one, two, three and more
 superblocks, so both buffers and the last step), against the dequantized
 weights in float64.
 
-The bar is derived: each input is x to 22 bits (2^-22), and the products of
+The bar is derived: each input is x to 22 bits (2^-22; Q4_K, whose record it
+is, the other formats hold every bit), and the products of
 a row are added in float32 in at most K / 16 + 24 roundings, each within
 2^-24 of the sum of the absolute products.
 """
@@ -117,9 +118,8 @@ def test_planes_infinite_inputs(gpu, orc, fmt, monkeypatch):
 
 
 def test_planes_parts_and_capture(gpu, orc):
-    """llmq_linear_noalloc over a scratch that holds part of the prompt's
-    record gives llmq_linear's bits; under graph capture, where the
-    context's workspace may not be kept, the replays stay within the bar."""
+    """llmq_linear_noalloc of a long prompt gives llmq_linear's bits; under
+    graph capture the replays stay within the bar."""
     torch, lm, ctx = gpu
     from llm_mojo_amd._lib import check as ok, lib
 
@@ -153,8 +153,8 @@ def test_planes_parts_and_capture(gpu, orc):
 
 
 def test_planes_two_streams(gpu, orc):
-    """Calls on alternating streams share the context's workspace: each gives
-    what it gives alone."""
+    """Calls on alternating streams of one context: each gives what it gives
+    alone."""
     torch, lm, ctx = gpu
     rng = np.random.default_rng(8)
     t, n, k = 512, 512, 4096

@@ -558,8 +558,14 @@ template <int HD, int RPW>
 int prompt_launch(llmq_ctx *ctx, const llmq_kv *kv, float *out, const float *qkv, int layer, int T, int pos0,
                   int64_t ld) {
     const int C = kv->n_head * kv->head_dim, n = pos0 + T;
-    // at most 49 KB, at 2048 positions of HD 128: 16 + 33
+    // at most 49 KB for HD 64 and 81 KB for HD 128, at 2048 positions: 16 of scales, 33 or 65 of sums
     const size_t lds = ((size_t)(n + kRun - 1) / kRun * kRun * 2 + (size_t)(n + 255) / 256 * 16 * (HD + 1)) * 4;
+    static size_t granted = 64 * 1024;
+    if (lds > granted) {
+        LLMQ_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&ikv_prompt_kernel<HD, RPW>),
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        granted = lds;
+    }
     hipLaunchKernelGGL((ikv_prompt_kernel<HD, RPW>), dim3(kv->n_head, (T + 15) / 16), dim3(64 * kPromptWaves), lds,
                        ctx->stream, qkv, ld ? ld : 3 * C, pos0, T, layer, kv->max_t, kv->n_head, kv->k, kv->v, kv->kq,
                        kv->vq, out, (int64_t)C, sqrt((double)HD));

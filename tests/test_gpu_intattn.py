@@ -71,6 +71,7 @@ PROMPT_EDGES = [
     (33, 479, 8, 64, 1.0), (33, 480, 8, 64, 1.0), (20, 1004, 13, 64, 1.0), (20, 1005, 13, 64, 1.0),  # runs a wave
     (40, 2008, 7, 64, 1.0), (40, 2009, 7, 64, 1.0),  # the longest context, and past it
     (16, 48, 16, 64, 1.0), (9, 120, 57, 128, 1.0), (65, 448, 8, 128, 1.0), (30, 1700, 18, 128, 1.0),
+    (30, 1506, 18, 128, 1.0), (30, 1507, 18, 128, 1.0), (30, 2018, 18, 128, 1.0),  # LDS about and past 64 KB, its most
     (19, 250, 14, 64, 0.0), (19, 250, 14, 64, 9000.0),  # equal scales; scales past int32
 ]
 

@@ -749,6 +749,7 @@ struct llmq_llama {
     int rows = 0;
     ArgmaxPart *hparts = nullptr;  // head argmax partials, batch x nhparts
     int nhparts = 0;               // the int16 head's partials a row, fixed at creation
+    int64_t one[2] = {0, 0};       // forward of one token: its token and position, until the copy is done
     float *apart = nullptr;        // decode attention split results, batch x heads x splits x kPart
     float2 *rope = nullptr;        // (cos, sin) of position p, pair i at [p * head_dim / 2 + i]
     float *x = nullptr, *xn = nullptr, *qkv = nullptr, *att = nullptr, *gu = nullptr, *hh = nullptr,
@@ -1060,9 +1061,10 @@ int llama_prefill(llmq_llama *m, int seq, const int64_t *tokens, int T, int pos0
     llmq_ctx *ctx = m->ctx;
     const llmq_llama_cfg &c = m->cfg;
     RC(ensure_rows(m, T));
-    const bool step = T == 1 && !pick;  // (forward, which waits for the copy of `one` before it returns)
-    const int64_t one[2] = {tokens[0], pos0};
-    LLMQ_HIP(hipMemcpyAsync(m->tokens, step ? one : tokens, sizeof(int64_t) * (step ? 2 : T), hipMemcpyHostToDevice,
+    const bool step = T == 1 && !pick;
+    m->one[0] = tokens[0];
+    m->one[1] = pos0;
+    LLMQ_HIP(hipMemcpyAsync(m->tokens, step ? m->one : tokens, sizeof(int64_t) * (step ? 2 : T), hipMemcpyHostToDevice,
                             ctx->stream));
     RC(launch_gguf_dequant_rows(ctx, m->embd, m->tokens, T, m->x, c.dim));
     RC(llama_layers(m, T, T, seq, pos0, step ? reinterpret_cast<const int *>(m->tokens + 1) : nullptr));

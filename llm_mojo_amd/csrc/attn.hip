@@ -50,10 +50,14 @@ __global__ __launch_bounds__(64) void kv_store_kernel(const float *__restrict__ 
 // head's new key and value (QuantKV.store, kvcache.mojo:333-342), writes them
 // to the cache, and uses them from LDS for the current position.
 //
-// What bounds it: one workgroup a head, so one CU's latency and the chains'
-// instructions.  MODE 2 against rows with a chain a lane, read by flat loads
-// (s_memtime cycles at 496 positions): total 7500 -> 2600, values 11400 ->
-// 6200, the whole kernel 16.2 -> ~11 us; GPT-2 decode after 476 tokens 410 ->
+// What bounds it: one workgroup a head, so one CU's latencies.  Of 21500
+// s_memtime cycles at 490 positions (one token, cached rows in L2) 5100 are
+// the first round trip (query, rows, scales), 4200 the scores and, beside
+// them, the waves' transposed stores, 1100 the maximum and the exponentials,
+// 4600 the total's chain, 600 the weights and 6200 the value chains: a wave
+// of a chain alone, the rest of the workgroup waiting.  MODE 2 against rows
+// with a chain a lane, read by flat loads: values 11400 -> 6200 cycles, the
+// whole kernel 16.2 -> ~11 us; GPT-2 decode after 476 tokens 410 ->
 // 352 us a token, after 900 541 -> 441, after 12 273 -> 264.  Values as fp16
 // columns for a mixed fma were slower (64 two-byte stores a position), a
 // chain of four lanes' quads too (its broadcast reads fill the LDS port), and
@@ -1041,21 +1045,22 @@ __device__ __forceinline__ float rows4_sum_p(float v) {
 // attend_prompt_kernel's attention for 4 of the 8 query heads of a key /
 // value head (workgroup x: key / value head, then which half of its heads) and
 // queries q0 .. q0 + 15 (q0 = 16 blockIdx.y) at once, on the fp16 matrix
-// cores: each staged block of 64 key / value rows serves them all.  Scores
-// k . q with the int8 codes exact in fp16 and q as hi / lo planes; a first pass over the keys finds each query's maximum and the
+// cores: each staged block of 64 key / value rows serves them all, a head a
+// wave.  Scores k . q with the int8 codes exact in fp16 and q as hi / lo
+// planes; a first pass over the keys finds each query's maximum and the
 // largest value scale, the second forms e = exp(s - max), the weights
 // e vs sigma as hi / lo planes (sigma a power of two, max vs sigma < 2^10)
-// and their products with the value codes.  Wave w owns R = 1
-// head: in the scores lane l holds query l % 16 and keys 4 (l / 16) + i of each
-// 16-key tile, which is the operand layout of the value products, so the
-// weights never leave registers.  Sums are in the matrix cores' order (float
-// rounding, not attend_prompt_kernel's bits).
+// and their products with the value codes.  In the scores lane l holds query
+// l % 16 and keys 4 (l / 16) + i of each 16-key tile, which is the operand
+// layout of the value products, so the weights never leave registers.  Sums
+// are in the matrix cores' order (float rounding, not attend_prompt_kernel's
+// bits).
 // What bounds it: a wave's own chain of blocks (exp and the weights' planes
 // most of its instructions) with few waves in flight: 4 key / value heads and
-// 400 tokens are 100 tiles of 8 heads.  Two heads a wave (R = 2, all 8 a
-// workgroup, the same bits) shared each staged block further and took 38.0 us
-// a layer against 23.4 at 400 tokens; a TinyLlama prompt of 128 tokens after
-// 1000 took 4.26 ms against 3.40, of 1900 tokens 16.7 against 16.1.
+// 400 tokens are 200 workgroups.  Two heads a wave (all 8 a workgroup, the
+// same bits) shared each staged block further and took 38.0 us a layer
+// against 23.4 at 400 tokens; a TinyLlama prompt of 128 tokens after 1000
+// took 4.26 ms against 3.40, of 1900 tokens 16.7 against 16.1.
 __global__ __launch_bounds__(256) void attend_prompt_gqa_kernel(const float *__restrict__ qkv, int64_t ld, int pos0,
                                                                 int T, int layer, int max_t, int n_kv,
                                                                 const int8_t *__restrict__ K8,
@@ -1063,43 +1068,40 @@ __global__ __launch_bounds__(256) void attend_prompt_gqa_kernel(const float *__r
                                                                 const float *__restrict__ KS,
                                                                 const float *__restrict__ VS, float *__restrict__ out,
                                                                 int64_t ldo, int hm) {
-    constexpr int HD = 64, G = 8, R = 1;       // head dim, heads a key / value head, heads a wave
-    constexpr int KR = HD + 8, VR = kPB + 4;   // LDS row strides (bytes)
+    constexpr int HD = 64, G = 8;             // head dim, heads a key / value head
+    constexpr int KR = HD + 8, VR = kPB + 4;  // LDS row strides (bytes)
     __shared__ __align__(16) int8_t kr[kPB][KR];
     __shared__ __align__(16) int8_t vt[HD][VR];
-    __shared__ float ksb[kPB], vsb[kPB], vmx[4], tfin[4][R][16];
+    __shared__ float ksb[kPB], vsb[kPB], vmx[4], tfin[4][16];
     const int kvh = blockIdx.x / 2, q0 = blockIdx.y * kQB, tid = threadIdx.x;
     const int lane = tid & 63, w = tid >> 6, c16 = lane & 15, g = lane >> 4;
-    const int h0 = kvh * G + 4 * R * ((int)blockIdx.x % 2) + R * w;  // the wave's first head
+    const int h = kvh * G + 4 * ((int)blockIdx.x % 2) + w;  // the wave's head
     const int nq = min(kQB, T - q0);
     const int npos = pos0 + q0 + nq;  // positions any query of the block sees
     const int64_t base = hm ? ((int64_t)layer * n_kv + kvh) * max_t : (int64_t)layer * max_t * n_kv + kvh;
     const int64_t pstr = hm ? 1 : n_kv;  // rows between positions
     const int qpos = pos0 + q0 + c16;  // the lane's query sees positions <= qpos
     const bool qok = c16 < nq;
-    // the query operand of head h0 + r: dims 32 kb + 8 g .., hi and lo planes
-    v8h bq[R][2][2];
+    // the query operand: dims 32 kb + 8 g .., hi and lo planes
+    v8h bq[2][2];
+    const float *qr = qkv + (int64_t)(q0 + c16) * ld + (int64_t)h * HD;
 #pragma unroll
-    for (int r = 0; r < R; r++) {
-        const float *qr = qkv + (int64_t)(q0 + c16) * ld + (int64_t)(h0 + r) * HD;
+    for (int kb = 0; kb < 2; kb++) {
+        float x[8];
 #pragma unroll
-        for (int kb = 0; kb < 2; kb++) {
-            float x[8];
+        for (int e = 0; e < 8; e += 4) {
+            float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            if (qok) v = *reinterpret_cast<const float4 *>(qr + 32 * kb + 8 * g + e);
+            x[e] = v.x;
+            x[e + 1] = v.y;
+            x[e + 2] = v.z;
+            x[e + 3] = v.w;
+        }
 #pragma unroll
-            for (int e = 0; e < 8; e += 4) {
-                float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                if (qok) v = *reinterpret_cast<const float4 *>(qr + 32 * kb + 8 * g + e);
-                x[e] = v.x;
-                x[e + 1] = v.y;
-                x[e + 2] = v.z;
-                x[e + 3] = v.w;
-            }
-#pragma unroll
-            for (int e = 0; e < 8; e++) {
-                const _Float16 hi = (_Float16)x[e];
-                bq[r][kb][0][e] = hi;
-                bq[r][kb][1][e] = (_Float16)(x[e] - (float)hi);
-            }
+        for (int e = 0; e < 8; e++) {
+            const _Float16 hi = (_Float16)x[e];
+            bq[kb][0][e] = hi;
+            bq[kb][1][e] = (_Float16)(x[e] - (float)hi);
         }
     }
     // Block s0's rows: thread (key tid / 4, piece tid % 4) loads 16 bytes of the
@@ -1137,26 +1139,21 @@ __global__ __launch_bounds__(256) void attend_prompt_gqa_kernel(const float *__r
         }
         __syncthreads();
     };
-    // scores of key tile kt of the staged block for head row tiles r: D[key 4 g + i][query c16]
-    auto scores = [&](int kt, v4f (&d)[R]) {
-#pragma unroll
-        for (int r = 0; r < R; r++) d[r] = (v4f){0.0f, 0.0f, 0.0f, 0.0f};
+    // scores of key tile kt of the staged block: D[key 4 g + i][query c16]
+    auto scores = [&](int kt) {
+        v4f d = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int kb = 0; kb < 2; kb++) {
             const uint2 kk = *reinterpret_cast<const uint2 *>(&kr[16 * kt + c16][32 * kb + 8 * g]);
             const v8h ak = s8x8_f16(kk.x, kk.y);
-#pragma unroll
-            for (int r = 0; r < R; r++) {
-                d[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ak, bq[r][kb][0], d[r], 0, 0, 0);
-                d[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ak, bq[r][kb][1], d[r], 0, 0, 0);
-            }
+            d = __builtin_amdgcn_mfma_f32_16x16x32_f16(ak, bq[kb][0], d, 0, 0, 0);
+            d = __builtin_amdgcn_mfma_f32_16x16x32_f16(ak, bq[kb][1], d, 0, 0, 0);
         }
+        return d;
     };
     const float scale = 1.0f / sqrtf((float)HD);
     // pass 1: each query's maximum, and the largest value scale
-    float mx[R], vm = 0.0f;
-#pragma unroll
-    for (int r = 0; r < R; r++) mx[r] = -INFINITY;
+    float mx = -INFINITY, vm = 0.0f;
     Rows nx = fetch(0, false);
     for (int s0 = 0; s0 < npos; s0 += kPB) {
         commit(nx, false);
@@ -1164,20 +1161,16 @@ __global__ __launch_bounds__(256) void attend_prompt_gqa_kernel(const float *__r
         if (s0 + kPB < npos) nx = fetch(s0 + kPB, false);
 #pragma unroll
         for (int kt = 0; kt < 4; kt++) {
-            v4f d[R];
-            scores(kt, d);
+            const v4f d = scores(kt);
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const int p = s0 + 16 * kt + 4 * g + i;
                 const float ks = ksb[16 * kt + 4 * g + i];
-#pragma unroll
-                for (int r = 0; r < R; r++)
-                    if (qok && p <= qpos) mx[r] = fmaxf(mx[r], d[r][i] * ks * scale);
+                if (qok && p <= qpos) mx = fmaxf(mx, d[i] * ks * scale);
             }
         }
     }
-#pragma unroll
-    for (int r = 0; r < R; r++) mx[r] = rows4_max_p(mx[r]);
+    mx = rows4_max_p(mx);
     vm = wave_max(vm);
     if (lane == 0) vmx[w] = vm;
     __syncthreads();
@@ -1185,36 +1178,29 @@ __global__ __launch_bounds__(256) void attend_prompt_gqa_kernel(const float *__r
     frexpf(fmaxf(fmaxf(vmx[0], vmx[1]), fmaxf(vmx[2], vmx[3])), &ex);
     const int sig_e = min(126, max(-126, 10 - ex));
     const float sigma = ldexpf(1.0f, sig_e);
-    // pass 2: weights and value sums; o[r][dt]: D[query 4 g + i][dim 16 dt + c16]
-    v4f o[R][4];
+    // pass 2: weights and value sums; o[dt]: D[query 4 g + i][dim 16 dt + c16]
+    v4f o[4];
 #pragma unroll
-    for (int r = 0; r < R; r++)
-#pragma unroll
-        for (int dt = 0; dt < 4; dt++) o[r][dt] = (v4f){0.0f, 0.0f, 0.0f, 0.0f};
-    float te[R] = {};
+    for (int dt = 0; dt < 4; dt++) o[dt] = (v4f){0.0f, 0.0f, 0.0f, 0.0f};
+    float te = 0.0f;
     nx = fetch(0, true);
     for (int s0 = 0; s0 < npos; s0 += kPB) {
         commit(nx, true);
         if (s0 + kPB < npos) nx = fetch(s0 + kPB, true);
-        v8h ph[R][2], pl[R][2];  // [r][key half]: element e is key 32 c + 16 (e / 4) + 4 g + e % 4
+        v8h ph[2], pl[2];  // [key half]: element e is key 32 c + 16 (e / 4) + 4 g + e % 4
 #pragma unroll
         for (int kt = 0; kt < 4; kt++) {
-            v4f d[R];
-            scores(kt, d);
+            const v4f d = scores(kt);
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const int p = s0 + 16 * kt + 4 * g + i;
                 const float ks = ksb[16 * kt + 4 * g + i], vs = vsb[16 * kt + 4 * g + i];
-#pragma unroll
-                for (int r = 0; r < R; r++) {
-                    const bool ok = qok && p <= qpos;
-                    const float e = ok ? expf(d[r][i] * ks * scale - mx[r]) : 0.0f;
-                    te[r] += e;
-                    const float x = e * vs * sigma;
-                    const _Float16 hi = (_Float16)x;
-                    ph[r][kt >> 1][4 * (kt & 1) + i] = hi;
-                    pl[r][kt >> 1][4 * (kt & 1) + i] = (_Float16)(x - (float)hi);
-                }
+                const float e = qok && p <= qpos ? expf(d[i] * ks * scale - mx) : 0.0f;
+                te += e;
+                const float x = e * vs * sigma;
+                const _Float16 hi = (_Float16)x;
+                ph[kt >> 1][4 * (kt & 1) + i] = hi;
+                pl[kt >> 1][4 * (kt & 1) + i] = (_Float16)(x - (float)hi);
             }
         }
 #pragma unroll
@@ -1224,34 +1210,25 @@ __global__ __launch_bounds__(256) void attend_prompt_gqa_kernel(const float *__r
                 const uint32_t v0 = *reinterpret_cast<const uint32_t *>(&vt[16 * dt + c16][32 * c + 4 * g]);
                 const uint32_t v1 = *reinterpret_cast<const uint32_t *>(&vt[16 * dt + c16][32 * c + 16 + 4 * g]);
                 const v8h bv = s8x8_f16(v0, v1);
-#pragma unroll
-                for (int r = 0; r < R; r++) {
-                    o[r][dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ph[r][c], bv, o[r][dt], 0, 0, 0);
-                    o[r][dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pl[r][c], bv, o[r][dt], 0, 0, 0);
-                }
+                o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ph[c], bv, o[dt], 0, 0, 0);
+                o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pl[c], bv, o[dt], 0, 0, 0);
             }
     }
     // each query's total, from the score layout (lane = query) to the value layout (4 g + i)
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-        te[r] = rows4_sum_p(te[r]);
-        if (g == 0) tfin[w][r][c16] = te[r];
-    }
+    te = rows4_sum_p(te);
+    if (g == 0) tfin[w][c16] = te;
     __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the wave's own LDS writes are in
     const float isig = ldexpf(1.0f, -sig_e);
 #pragma unroll
-    for (int r = 0; r < R; r++)
+    for (int i = 0; i < 4; i++) {
+        const int q = 4 * g + i;
+        if (q < nq) {
+            const float t = tfin[w][q];
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int q = 4 * g + i;
-            if (q < nq) {
-                const float t = tfin[w][r][q];
-#pragma unroll
-                for (int dt = 0; dt < 4; dt++)
-                    out[(int64_t)(q0 + q) * ldo + (int64_t)(h0 + r) * HD + 16 * dt + c16] =
-                        o[r][dt][i] * isig / t;
-            }
+            for (int dt = 0; dt < 4; dt++)
+                out[(int64_t)(q0 + q) * ldo + (int64_t)h * HD + 16 * dt + c16] = o[dt][i] * isig / t;
         }
+    }
 }
 
 }  // namespace

@@ -15,8 +15,9 @@
 static thread_local char g_err[512];
 
 // The scratch of llmq_linear_noalloc: the prompt GEMM's int16 activation
-// codes (256-byte aligned) and per-row scales, which llmq_linear keeps in the
-// context's grow-only workspace.  Each GPU the library runs on holds its own
+// codes (256-byte aligned), per-row scales and fp16 planes and the Q4_K
+// matmul's record, which llmq_linear keeps in the context's grow-only
+// workspaces.  Each GPU the library runs on holds its own
 // copy for the life of the process.  The array's name is a host-side stand-in
 // (never passed to a kernel): host code uses the device address that
 // hipGetSymbolAddress returns, looked up once per device by llmq_init.

@@ -36,7 +36,7 @@ struct llmq_ctx {
     hipDeviceProp_t prop{};
     // grow-only workspaces: slot 0 the prompt-side int16 activation codes
     // (and LayerNorm outputs), slot 1 the fp16 activation records of the
-    // several-token float-activation matmul
+    // several-token Q4_K matmul
     void *ws[2] = {nullptr, nullptr};
     size_t ws_bytes[2] = {0, 0};
     hipStream_t ws_stream = nullptr;  // the stream that used a workspace last
@@ -276,7 +276,8 @@ int gemv_a16_num_parts(const llmq_mat *w, bool ln);
 bool gemv1_supports(const llmq_mat *w, bool ln);
 // The prompt-side int8-MFMA GEMM (gemm_mfma.hip): xq / sx are T x K int16
 // codes and T scales of workspace; with `planes` (gemm_f16_planes_bytes of
-// workspace, for matrices gemm_f16_supports takes: int4 in groups of 32)
+// workspace, for matrices gemm_f16_supports takes: groups of 32, or whole
+// 256-input superblocks whose groups are a power of two times 32 or the row)
 // the codes also go there as fp16 planes and the fp16 matrix-core form runs.
 bool gemm_mfma_supports(const llmq_mat *w, int64_t T);
 bool gemm_f16_supports(const llmq_mat *w, int64_t T);

@@ -853,8 +853,11 @@ int launch_gemm_mfma(llmq_ctx *ctx, const GemvRequest &rq, int16_t *xq, float *s
     const int full = (int)(w->n / 32 * 32);
     // gemm_planes.hip's tiles, except where the 16 x 64 tile of
     // gemm_f16_kernel is the faster one: int4 in groups of 32 with fewer than
-    // 640 workgroups of 32 x 64 (301 x 3072 x 768 21.2 us here, 23.3 there;
-    // 476 x 768 x 3072 15.9 and 14.8; int8 27.9 and 23.3, 18.6 and 17.6)
+    // 640 workgroups of 32 x 64.  Of 129 shapes (2 to 1024 tokens, 768 to
+    // 8192 inputs, 768 to 12000 rows) it took 6 % less than there in the mean
+    // of the 98 below that line (84 to 103 % of the other's time), 5 % more
+    // in the mean of the 31 above (85 to 128 %); int8 301 x 3072 x 768 27.9
+    // and 23.3 us, 476 x 768 x 3072 18.6 and 17.6
     const bool big = (T + 31) / 32 * ((full + 63) / 64) >= 640;
     if (planes && full > 0 && !rq.kv && gemm_planes_a16_ok(w) && !(w->group == 32 && getenv("LLMQ_F16_TILE")) &&
         (w->group != 32 || w->bits == 8 || big)) {

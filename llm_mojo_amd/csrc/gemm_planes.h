@@ -867,8 +867,7 @@ __global__ __launch_bounds__(WT * WR * WK * 64, Tr<F>::F32 ? 4 : 2) void gemm_pl
     }
 }
 
-// The tiles, as TT, RT, WT, WR, WK, S (kTiles in gemm_planes.hip has
-// what each costs).
+// The tiles, as TT, RT, WT, WR, WK, S (gemm_planes.hip has what each costs).
 template <int F, int SEG>
 int launch_tile(hipStream_t st, int tile, const Args &a) {
     const int tt = (a.T + 15) / 16, rt = a.ntiles;

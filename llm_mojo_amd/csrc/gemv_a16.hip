@@ -499,8 +499,8 @@ int launch_gemv_a16(llmq_ctx *ctx, const GemvRequest &rq) {
         int min_t = exact_order() ? 2 : 8;
         if (const char *e = getenv("LLMQ_MFMA_MIN_T")) min_t = atoi(e);
         if (rq.T >= min_t && min_t > 0 && gemm_mfma_supports(w, rq.T)) {
-            // workspace: int16 codes, token scales, then (int4-g32) the fp16
-            // planes; a caller-given workspace too small for the planes runs
+            // workspace: int16 codes, token scales, then (gemm_f16_supports) the
+            // fp16 planes; a caller-given workspace too small for the planes runs
             // the int8-MFMA form, whose results are the same bits
             const size_t xb = ((size_t)rq.T * w->k * 2 + 255) & ~(size_t)255;
             const size_t sb = ((size_t)rq.T * 4 + 255) & ~(size_t)255;

@@ -10,9 +10,9 @@
 // exponents): v_mfma_f32_16x16x32_bf16 forms sum q (p0 + p1 + p2) with every
 // product exact in its fp32 sums.  So a call needs no memory and no other
 // kernel, an input (from 2^-110 on) keeps its last bit whatever its neighbours
-// are, and what is left of the format is applied in fp32: the block's scale per chunk of
-// 32 inputs (Q8_0, Q4_0, Q4_1, Q5_K's sub-blocks, groups of 32 to 128) or per
-// 4 chunks or superblock of 8 (Q6_K, one scale a row).  Q6_K's codes times
+// are, and what is left of the format is applied in fp32: the block's scale
+// per chunk of 32 inputs (Q8_0, Q4_0, Q4_1, Q5_K's sub-blocks, groups of 32 to
+// 128) or per superblock of 8 (Q6_K, one scale a row).  Q6_K's codes times
 // their sub-block scale are 13 bits: two bf16 operands.  Q4_1 and Q5_K take
 // their codes less 8 or 16 and the rest of the offset times the chunk's sum
 // of x, both in fp32 (the sum on the fp32 matrix cores), which keeps the two
@@ -20,8 +20,8 @@
 // (an infinity, a NaN, inputs from 2^100 on, or nothing above 2^-85) are left
 // out of the planes and added to the outputs weight by weight at the end.
 // Off the 64-bit result (476 x 768 x 2304, a residual stream; the fp32 matrix
-// cores): Q8_0 0.8e-7 (2.9e-7), Q5_K 0.9e-7 (2.9e-7), Q6_K 1.4e-7 (2.9e-7),
-// int8-ch 1.1e-7 (2.9e-7).  Two fp16 planes under an exponent a superblock
+// cores): Q8_0 1.0e-7 (2.9e-7), Q5_K 1.0e-7 (2.9e-7), Q6_K 1.2e-7 (2.9e-7),
+// int8-ch 1.0e-7 (2.9e-7).  Two fp16 planes under an exponent a superblock
 // (22 bits, Q4_K's record below) were as close there and took 2 products for
 // 3, but lost a small input beside one 2^20 times as large, to all of it.
 //
@@ -48,17 +48,17 @@
 // 16 cycles and ~15 vector instructions of 4 (7 decode its share of a row
 // tile's codes, 4 scale it, 4 to 5 split its share of x), and each wave reads
 // 3 KB of planes a token tile and chunk.  512 x 4096 x 11008 Q8_0 in the
-// widest tile: matrix cores busy 31 % of the time, the vector units 49 %, LDS
-// 25 % (counters), the rest waits at 4 waves a SIMD; 16 waves a CU that split
-// for 256 rows did more than wider wave tiles at 8 (4 x 2: 218 us, 2 x 4: 223,
-// 2 x 2 as here: 166).  Few workgroups are bound by a wave's own chain through
+// 256-row tile: matrix cores busy 34 % of the time, the vector units 53 %, LDS
+// 35 % (counters), the rest waits at 4 waves a SIMD; 16 waves a CU did more
+// than wider wave tiles at 8 (4 x 2: 218 us, 2 x 4: 223, 2 x 2: 166, 2 x 3 in
+// 128 registers: 157).  Few workgroups are bound by a wave's own chain through
 // a step (~1 us for 2 chunks): tiles whose waves share the chunks out (WK = 2,
 // 4).  Over a record, the LDS reads take half of the products' time and the
 // decode and scales come to their own time at TT = 2; three or four buffers
 // in flight instead of two measured the same or slower at every size.
-// 512 x 4096 x 11008, fp32 matrix cores and here: Q8_0 1059 us and 165, Q4_0
-// 1134 and 161, Q4_1 1134 and 184, Q5_K 777 and 200, Q6_K 1168 and 265,
-// int8-ch 1142 and 175, int4-g32 1148 and 173 (0.84 PFLOP/s of bf16 products
+// 512 x 4096 x 11008, fp32 matrix cores and here: Q8_0 1059 us and 157, Q4_0
+// 1134 and 161, Q4_1 1134 and 187, Q5_K 777 and 202, Q6_K 1168 and 274,
+// int8-ch 1142 and 182, int4-g32 1148 and 165 (0.88 PFLOP/s of bf16 products
 // at Q8_0); Q4_K 725 and 124 with its record.
 //
 // int16 activation codes (kA4, kA8) come as two exact planes of their own,
@@ -202,8 +202,8 @@ __device__ float weight(const Args &a, int rt, int r, int c, int k) {
     return 0.0f;
 }
 
-// SEG: chunks of 32 inputs that share a scale (1, 2, 4, or 8 for one scale a
-// superblock or more).
+// SEG0: chunks of 32 inputs that share a scale (1, 2, 4, or 8 for one scale a
+// superblock or more; over floats 1 or 8).
 template <int F, int SEG0, int TT, int RT, int WT, int WR, int WK, int S>
 __global__ __launch_bounds__(WT * WR * WK * 64, Tr<F>::F32 ? 4 : 2) void gemm_planes_kernel(Args a) {
     using R = Tr<F>;
@@ -211,12 +211,10 @@ __global__ __launch_bounds__(WT * WR * WK * 64, Tr<F>::F32 ? 4 : 2) void gemm_pl
     constexpr int SPB = 8 / S;  // steps a superblock
     static_assert(8 % S == 0 && S % WK == 0 && 4 % WK == 0, "whole steps a superblock, chunks for every wave");
     constexpr int NW = WT * WR * WK, RB = NW * 1024;  // bytes a copy round: 16 a lane
-    // (waves that share a group's chunks scale each by itself)
-    constexpr int SEG = WK > 1 && SEG0 < 8 ? 1 : SEG0;
-    // One scale a superblock: the products of its chunks chain, over floats a wave's of at most 4 at a time
-    // (of all 8, 48 roundings at the sum's size put Q6_K 2.0e-7 off the 64-bit result at 476 x 768 x 2304).
-    constexpr bool HALF = R::F32 && F != kQ5_K && (R::KQ || SEG == 8), CHAIN = F == kQ4_K || HALF;
-    constexpr int RUN = WK == 1 ? 4 : 8;  // chunks of such a chain, WK waves' together
+    constexpr int SEG = R::F32 ? 1 : SEG0;  // (over floats every chunk's sums are scaled or added by themselves)
+    // One scale a superblock: over a record the products of its chunks chain, over floats, with twice as many
+    // and more of Q6_K, the chunks' sums are added (chained, Q6_K was 2.0e-7 off at 476 x 768 x 2304).
+    constexpr bool CHAIN = F == kQ4_K, ONE = R::F32 && F != kQ5_K && (R::KQ || SEG0 == 8);
     // separate arrays, so that the compiler sees a copy into one cannot alias reads of another
     __shared__ __align__(16) uint8_t b0[L::STEP], b1[L::STEP], f0[L::SBUF ? L::SBUF : 16], f1[L::SBUF ? L::SBUF : 16];
     // F32: the step's planes, the superblock's sums of x a chunk, and which token tiles have inputs left out of the planes
@@ -434,12 +432,12 @@ __global__ __launch_bounds__(WT * WR * WK * 64, Tr<F>::F32 ? 4 : 2) void gemm_pl
     for (int t = 0; t < TT; t++)
 #pragma unroll
         for (int r = 0; r < RT; r++) acc[t][r] = zero;
-    v4f seg[TT][RT], sel[TT][RT];   // SEG > 1: the group's sums (A16: of the hi and the lo plane)
+    v4f seg[TT][RT], sel[TT][RT];   // A16, SEG > 1: the group's sums of the hi and the lo plane
     v2h sc[RT][4];                  // Q4_K: sub-block scales (sc_2i, sc_2i+1)
     uint32_t sl5[RT], sh5[RT];      // Q5_K: the same as bytes, 0-3 and 4-7
     uint32_t mp[RT][4];             // Q4_K: minima of the 8 chunks, fp16 pairs
     float cm[RT][2] = {};           // CENTER: the offsets of chunks g and 4 + g
-    float rs[RT];                   // HALF: the row's scale
+    float rs[RT];                   // ONE: the row's scale
 
     // this lane's place in each region of a buffer (opaque, so that a read is one step from its buffer)
     auto place = [](int v) { asm("" : "+v"(v)); return v; };
@@ -453,17 +451,17 @@ __global__ __launch_bounds__(WT * WR * WK * 64, Tr<F>::F32 ? 4 : 2) void gemm_pl
     const int pU = place(R::CENTER ? wt * TT * 512 + c16 * 32 + g * 4 : L::oSU + wt * TT * 512 + (lane & 31) * 16);
     const int pI = place(L::oIV + wt * TT * 64 + g * 16);
 
-    // row tile r's sums x of chunk j (or of its group, at the last) times the scale s
+    // F32: row tile r's sums x of chunk j, times the scale s unless that is the superblock's
     auto scale = [&](int j, int r, const v4f (&x)[TT], float s) __attribute__((always_inline)) {
 #pragma unroll
         for (int t = 0; t < TT; t++) {
-            if (SEG == 1 || (j + 1) % SEG == 0) {
 #pragma unroll
-                for (int i = 0; i < 4; i++) d[t][r][i] = j < SEG ? s * x[t][i] : fmaf(s, x[t][i], d[t][r][i]);
-                asm volatile("" : "+v"(d[t][r]));  // (formed here: sunk past a branch, its products' results would pile up)
-            } else {
-                seg[t][r] = x[t];
-            }
+            for (int i = 0; i < 4; i++)
+                if constexpr (ONE)
+                    d[t][r][i] = j == 0 ? x[t][i] : d[t][r][i] + x[t][i];
+                else
+                    d[t][r][i] = j == 0 ? s * x[t][i] : fmaf(s, x[t][i], d[t][r][i]);
+            asm volatile("" : "+v"(d[t][r]));  // (formed here: sunk past a branch, its products' results would pile up)
         }
     };
 
@@ -512,10 +510,12 @@ __global__ __launch_bounds__(WT * WR * WK * 64, Tr<F>::F32 ? 4 : 2) void gemm_pl
                 for (int q = 0; q < (R::F32 ? 3 : 2); q++)
                     ap[t][q] = lds<uint4>(R::F32 ? xb : cur, pA + (t * S + u) * R::AB + q * 1024);
             // F32: with them the chunk's codes and scales, so that the wave waits once (512 x 4096 x 11008
-            // Q8_0 in the widest tile: 175 us with the reads where they are used, 166 so)
+            // Q8_0 in the 256-row tile: 175 us with the reads where they are used, 166 so; the widest has no
+            // registers for it)
             uint2 cv[RT];
             uint32_t sv[RT], zv[RT];
-            if constexpr (R::F32) {
+            constexpr bool EARLY = R::F32 && RT < 3;
+            if constexpr (EARLY) {
 #pragma unroll
                 for (int r = 0; r < RT; r++) {
                     const int e = r * S + u;
@@ -538,11 +538,11 @@ __global__ __launch_bounds__(WT * WR * WK * 64, Tr<F>::F32 ? 4 : 2) void gemm_pl
                 uint32_t ev = 0, od = 0;
                 uint2 cw = {};
                 if constexpr (R::W8) {
-                    cw = R::F32 ? cv[r] : lds<uint2>(cur, pC + e * 512);
+                    cw = EARLY ? cv[r] : lds<uint2>(cur, pC + e * 512);
                     ev = __builtin_amdgcn_perm(cw.y, cw.x, 0x06040200u);
                     od = __builtin_amdgcn_perm(cw.y, cw.x, 0x07050301u);
                 } else {
-                    const uint32_t c4 = R::F32 ? cv[r].x : lds<uint32_t>(cur, pC + e * 256);
+                    const uint32_t c4 = EARLY ? cv[r].x : lds<uint32_t>(cur, pC + e * 256);
                     ev = c4 & 0x0F0F0F0Fu;
                     od = (c4 >> 4) & 0x0F0F0F0Fu;
                 }
@@ -581,7 +581,7 @@ __global__ __launch_bounds__(WT * WR * WK * 64, Tr<F>::F32 ? 4 : 2) void gemm_pl
                             }
                         } else {
                             float z = F == kQ5_K ? -1040.0f : -1032.0f;
-                            if constexpr (R::QM) z = -1024.0f - (float)zv[r];
+                            if constexpr (R::QM) z = -1024.0f - (float)(EARLY ? zv[r] : lds<uint8_t>(cur, pZ + e * 16));
 #pragma unroll
                             for (int i = 0; i < 4; i++) halves_add(q[i], z, f[2 * i], f[2 * i + 1]);
                         }
@@ -615,15 +615,15 @@ __global__ __launch_bounds__(WT * WR * WK * 64, Tr<F>::F32 ? 4 : 2) void gemm_pl
                 const v8h b = __builtin_bit_cast(v8h, bw);
                 float s = 0.0f;
                 if constexpr (F == kQ4_1) {
-                    const uint32_t m = sv[r];
+                    const uint32_t m = EARLY ? sv[r] : lds<uint32_t>(cur, pS + e * 64);
                     s = h2f(m & 0xFFFFu);
                     const float c = fmaf(8.0f, s, h2f(m >> 16));  // lane group j % 4 keeps chunk j's
                     cm[r][j >> 2] = (j & 3) + kk == g ? c : cm[r][j >> 2];
                 } else if constexpr (F == kQ5_K) {
                     s = (float)(((j < 4 ? sl5[r] : sh5[r]) >> (8 * (j & 3))) & 255u);
                 } else if constexpr (!R::KQ) {
-                    if ((j + WK) % (HALF ? RUN : SEG) == 0) s = h2f(R::F32 ? sv[r] : lds<uint16_t>(cur, pS + e * 32));
-                    if (HALF && (j + WK) % RUN == 0) rs[r] = s;
+                    if (R::F32 ? !ONE || j + WK == 8 : (j + 1) % SEG == 0) s = h2f(EARLY ? sv[r] : lds<uint16_t>(cur, pS + e * 32));
+                    if (ONE && j + WK == 8) rs[r] = s;
                 }
                 if constexpr (R::A16) {
                     // sum 256 hi w and sum lo w over the group's chunks (256 inputs at most), each exact
@@ -656,18 +656,25 @@ __global__ __launch_bounds__(WT * WR * WK * 64, Tr<F>::F32 ? 4 : 2) void gemm_pl
                 v4f x[TT];
 #pragma unroll
                 for (int t = 0; t < TT; t++)
-                    x[t] = CHAIN ? (j == 0 || (HALF && j % RUN == 0) ? zero : d[t][r]) : (j % SEG == 0 ? zero : seg[t][r]);
+                    x[t] = CHAIN && j > 0 ? d[t][r] : zero;
                 if constexpr (R::F32) {
-                    auto product = [&](const uint4 &wb) __attribute__((always_inline)) {  // smallest first
+                    // Largest first: what a product is added to, the matrix cores round to nearest where it is
+                    // the larger, but cut downwards where it is the smaller (smallest first left a mean error of
+                    // -0.9e-7 of the results' size at 301 x 4096 x 1000; so -1e-9).
+                    auto product = [&](int q, const uint4 &wb) __attribute__((always_inline)) {
 #pragma unroll
-                        for (int q = 2; q >= 0; q--)
-#pragma unroll
-                            for (int t = 0; t < TT; t++)
-                                x[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                                    __builtin_bit_cast(v8b, ap[t][q]), __builtin_bit_cast(v8b, wb), x[t], 0, 0, 0);
+                        for (int t = 0; t < TT; t++)
+                            x[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8b, ap[t][q]),
+                                                                           __builtin_bit_cast(v8b, wb), x[t], 0, 0, 0);
                     };
-                    if constexpr (F == kQ6_K) product(be);
-                    product(bw);
+                    product(0, bw);
+                    product(1, bw);
+                    if constexpr (F == kQ6_K) product(0, be);
+                    product(2, bw);
+                    if constexpr (F == kQ6_K) {
+                        product(1, be);
+                        product(2, be);
+                    }
                 } else {
 #pragma unroll
                     for (int q = 0; q < 2; q++)
@@ -689,20 +696,8 @@ __global__ __launch_bounds__(WT * WR * WK * 64, Tr<F>::F32 ? 4 : 2) void gemm_pl
                     if (r + 1 == RT) scale(j, r, px, ps);
                 }
             }
-            if constexpr (HALF) {
-                if ((j + WK) % RUN == 0) {
-#pragma unroll
-                    for (int r = 0; r < RT; r++) {
-                        if constexpr (F == kQ6_K) rs[r] = h2f(lds<uint16_t>(sbf, pD + r * 32));
-#pragma unroll
-                        for (int t = 0; t < TT; t++)
-#pragma unroll
-                            for (int i = 0; i < 4; i++) acc[t][r][i] = fmaf(rs[r], d[t][r][i], acc[t][r][i]);
-                    }
-                }
-            }
         }
-        if constexpr (j0 + S == 8 && !R::A16 && !HALF) {  // the superblock's minima, scale and 1 / s
+        if constexpr (j0 + S == 8 && !R::A16) {  // the superblock's minima, scale and 1 / s
             float dd[RT], dmin[RT];
             v8h bm[RT];
 #pragma unroll
@@ -713,6 +708,8 @@ __global__ __launch_bounds__(WT * WR * WK * 64, Tr<F>::F32 ? 4 : 2) void gemm_pl
                     const uint32_t f = lds<uint32_t>(sbf, pF + r * 256);
                     dd[r] = h2f(f & 0xFFFFu);
                     dmin[r] = -h2f(f >> 16);
+                } else if constexpr (F == kQ6_K) {
+                    rs[r] = h2f(lds<uint16_t>(sbf, pD + r * 32));
                 }
                 if constexpr (F == kQ4_K) {  // the minima in groups 0 and 1, against the sums' hi and lo planes
 #pragma unroll
@@ -753,7 +750,8 @@ __global__ __launch_bounds__(WT * WR * WK * 64, Tr<F>::F32 ? 4 : 2) void gemm_pl
                             v = fmaf(dd[r], v, dm[i]);
                         else if constexpr (F == kQ4_1)
                             v += dm[i];
-                        acc[t][r][i] = R::F32 ? acc[t][r][i] + v : fmaf(iv[i], v, acc[t][r][i]);
+                        acc[t][r][i] = ONE ? fmaf(rs[r], v, acc[t][r][i])
+                                           : R::F32 ? acc[t][r][i] + v : fmaf(iv[i], v, acc[t][r][i]);
                     }
                 }
             }
@@ -886,10 +884,16 @@ int launch_tile(hipStream_t st, int tile, const Args &a) {
         return LLMQ_OK;
     } else if constexpr (Tr<F>::F32) {
         switch (tile) {
-        case 0: LLMQ_PK(2, 2, 1, 8, 1, 2); break;
-        case 1: LLMQ_PK(2, 1, 1, 8, 2, 4); break;
-        case 2: LLMQ_PK(1, 2, 1, 4, 4, 8); break;
-        case 3: LLMQ_PK(1, 1, 1, 4, 4, 8); break;
+        case 0:  // (only where 128 registers hold it)
+            if constexpr (Tr<F>::KQ || Tr<F>::CENTER || SEG == 8)
+                LLMQ_PK(2, 2, 1, 8, 1, 2);
+            else
+                LLMQ_PK(2, 3, 1, 8, 1, 2);
+            break;
+        case 1: LLMQ_PK(2, 2, 1, 8, 1, 2); break;
+        case 2: LLMQ_PK(2, 1, 1, 8, 2, 4); break;
+        case 3: LLMQ_PK(1, 2, 1, 4, 4, 8); break;
+        case 4: LLMQ_PK(1, 1, 1, 4, 4, 8); break;
         default: LLMQ_PK(1, 1, 1, 2, 4, 8); break;
         }
     } else {

@@ -67,47 +67,63 @@ static int forced_tile() {
     return t < 0 ? 0 : t > 6 ? 6 : t;
 }
 
-// Q4_K's tile, the one with the least time by kTiles' figures (few tokens
-// have a kernel of their own).
-static int q4k_tile(const llmq_mat *w, int64_t T) {
+// The tile from `first` on with the least time by kTiles' figures, and that time.
+static int least_tile(const llmq_mat *w, int64_t T, int first, float *us) {
     using namespace planes;
-    int best = forced_tile();
-    if (best >= 0) return best;
-    float least = 0.0f;
-    for (int i = 0; i < (int)(sizeof(kTiles) / sizeof(kTiles[0])); i++) {
-        const float us = tile_us(kTiles[i], (T + 15) / 16, w->ntiles, w->k);
-        if (best < 0 || us < least) {
+    int best = first;
+    *us = tile_us(kTiles[first], (T + 15) / 16, w->ntiles, w->k);
+    for (int i = first + 1; i < (int)(sizeof(kTiles) / sizeof(kTiles[0])); i++) {
+        const float t = tile_us(kTiles[i], (T + 15) / 16, w->ntiles, w->k);
+        if (t < *us) {
             best = i;
-            least = us;
+            *us = t;
         }
     }
     return best;
 }
 
-// The tiles over floats: what a superblock costs in microseconds with one
-// workgroup on the fullest of the 256 CUs, and each further one there; 4 us
-// before the first.  Fitted to 237 calls of Q8_0, int4-g32 and int8-ch (16
-// to 1024 tokens, 768 to 8192 inputs, 768 to 12000 rows), 6 to 12 % off a
-// tile's times.  The fp32 kernel does 22 MAC a picosecond (16 tokens of 4096
-// x 4096: 13 us against 16; 64 tokens 50 against 18).  With these the choice
-// is within 1 % of the best of the six on all of those calls, and within 9 %
-// on 79 of Q6_K, whose products are twice as many.
+// Q4_K's tile (few tokens have a kernel of their own).
+static int q4k_tile(const llmq_mat *w, int64_t T) {
+    const int forced = forced_tile();
+    float us;
+    return forced >= 0 ? forced : least_tile(w, T, 0, &us);
+}
+
+// The tiles over floats (the widest only where the kernel has it): what a
+// superblock costs in microseconds with one workgroup on the fullest of the
+// 256 CUs, and each further one there.  Fitted to 237 calls of Q8_0, int4-g32
+// and int8-ch (16 to 1024 tokens, 768 to 8192 inputs, 768 to 12000 rows), 6
+// to 12 % off a tile's times and within 1 % of the best of them by the choice;
+// within 10 % on 79 of Q6_K, whose products are twice as many.
+//
+// The fp32 kernel (22 MAC a picosecond) is further off the 64-bit result, so
+// it has only what it is the clearly faster one for: the line lies at 4 us
+// and the least of kTiles' times, a little above the times here (10 x 1280 x
+// 7224 Q4_1, near it: 7.3 us and 3.6e-7 off there, 8.2 and 1.0e-7 here; 16
+// tokens of 4096 x 4096 Q8_0 12.2 us there and 16.8 here, 64 tokens 50 and
+// 18.5).
 int gemm_floats_tile(const llmq_mat *w, int64_t T) {
     using namespace planes;
     struct FloatTile {
         int tt, rt;
         float us, more;
     };
-    static constexpr FloatTile tiles[] = {{2, 16, 4.10f, 3.33f}, {2, 8, 2.53f, 3.17f}, {1, 8, 1.60f, 2.06f},
-                                          {1, 4, 1.02f, 1.28f},  {1, 2, 0.73f, 0.69f}};
+    static constexpr FloatTile tiles[] = {{2, 24, 5.88f, 4.66f}, {2, 16, 4.09f, 3.31f}, {2, 8, 2.53f, 3.17f},
+                                          {1, 8, 1.60f, 2.06f},  {1, 4, 1.02f, 1.27f},  {1, 2, 0.74f, 0.70f}};
     int best = forced_tile();
     if (best >= 0) return best;
-    float least = 2.5f + (float)T * (float)w->k * (float)w->n / 22e6f;
-    for (int i = 0; i < (int)(sizeof(tiles) / sizeof(tiles[0])); i++) {
+    int seg = 1, shift;
+    if (w->kind == MAT_QUANT) qm_groups(w, &seg, &shift);
+    const int ty = float_act_type(w);
+    const bool wide = w->kind == MAT_QUANT ? seg < 8 : ty == LLMQ_GGML_Q8_0 || ty == LLMQ_GGML_Q4_0;
+    float least;
+    least_tile(w, T, wide || ty == LLMQ_GGML_Q4_1 ? 1 : 0, &least);
+    if (3.5f + (float)T * (float)w->k * (float)w->n / 22e6f < 4.0f + least) return -1;
+    for (int i = wide ? 0 : 1; i < (int)(sizeof(tiles) / sizeof(tiles[0])); i++) {
         const FloatTile &k = tiles[i];
         const int64_t wgs = ((T + 15) / 16 + k.tt - 1) / k.tt * ((w->ntiles + k.rt - 1) / k.rt);
-        const float us = 4.0f + (float)(w->k / 256) * (k.us + k.more * (float)((wgs + 255) / 256 - 1));
-        if (us < least) {
+        const float us = k.us + k.more * (float)((wgs + 255) / 256 - 1);
+        if (best < 0 || us < least) {
             best = i;
             least = us;
         }

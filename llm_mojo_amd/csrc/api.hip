@@ -76,6 +76,7 @@ bool ws_record(llmq_ctx *ctx) {
 // stream left while it was being captured is waited for from the capture's
 // end on.
 int ws_take(llmq_ctx *ctx) {
+    if (ctx->ws_stream == ctx->stream && !ctx->ws_recorded) return LLMQ_OK;  // in order by itself
     if (capturing(ctx->stream)) return LLMQ_OK;
     if (ctx->ws_stream && (ctx->ws_stream != ctx->stream || ctx->ws_recorded) && ws_record(ctx))
         LLMQ_HIP(hipStreamWaitEvent(ctx->stream, ctx->ws_event, 0));

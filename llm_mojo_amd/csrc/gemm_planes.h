@@ -503,12 +503,19 @@ __global__ __launch_bounds__(WT * WR * WK * 64, Tr<F>::F32 ? 4 : 2) void gemm_pl
             const int j = j0 + u;  // this wave's chunk is j + kk
             v4f px[TT];
             float ps = 0.0f;
-            uint4 ap[TT][R::F32 ? 3 : 2];
+            // (one array for either kind cost the record's kernels up to 20 more waits in the compiler's schedule)
+            uint4 ap[TT][3], ah[TT], al[TT];
 #pragma unroll
-            for (int t = 0; t < TT; t++)
+            for (int t = 0; t < TT; t++) {
+                const int p = pA + (t * S + u) * R::AB;
+                if constexpr (R::F32) {
 #pragma unroll
-                for (int q = 0; q < (R::F32 ? 3 : 2); q++)
-                    ap[t][q] = lds<uint4>(R::F32 ? xb : cur, pA + (t * S + u) * R::AB + q * 1024);
+                    for (int q = 0; q < 3; q++) ap[t][q] = lds<uint4>(xb, p + q * 1024);
+                } else {
+                    ah[t] = lds<uint4>(cur, p);
+                    al[t] = lds<uint4>(cur, p + 1024);
+                }
+            }
             // F32: with them the chunk's codes and scales, so that the wave waits once (512 x 4096 x 11008
             // Q8_0 in the 256-row tile: 175 us with the reads where they are used, 166 so; the widest has no
             // registers for it)
@@ -559,7 +566,8 @@ __global__ __launch_bounds__(WT * WR * WK * 64, Tr<F>::F32 ? 4 : 2) void gemm_pl
                     ev |= ((y << 4) & 0x00300030u) | ((y << 8) & 0x30003000u);
                     od |= ((y << 2) & 0x00300030u) | ((y << 6) & 0x30003000u);
                 }
-                uint4 bw, be;  // the weights as 16-bit floats; Q6_K: and what bf16 leaves of sc q
+                v8h b;         // the weights in fp16
+                uint4 bw, be;  // F32: in bf16; Q6_K: and what bf16 leaves of sc q
                 if constexpr (R::F32) {
                     float f[8];
                     if constexpr (F == kQ8_0) {
@@ -609,10 +617,12 @@ __global__ __launch_bounds__(WT * WR * WK * 64, Tr<F>::F32 ? 4 : 2) void gemm_pl
 #pragma unroll
                         for (int i = 0; i < 4; i++) q[i] = q[i] - z;
                     }
-                    bw = make_uint4(__builtin_bit_cast(uint32_t, q[0]), __builtin_bit_cast(uint32_t, q[1]),
-                                    __builtin_bit_cast(uint32_t, q[2]), __builtin_bit_cast(uint32_t, q[3]));
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        b[2 * i] = q[i][0];
+                        b[2 * i + 1] = q[i][1];
+                    }
                 }
-                const v8h b = __builtin_bit_cast(v8h, bw);
                 float s = 0.0f;
                 if constexpr (F == kQ4_1) {
                     const uint32_t m = EARLY ? sv[r] : lds<uint32_t>(cur, pS + e * 64);
@@ -623,7 +633,7 @@ __global__ __launch_bounds__(WT * WR * WK * 64, Tr<F>::F32 ? 4 : 2) void gemm_pl
                     s = (float)(((j < 4 ? sl5[r] : sh5[r]) >> (8 * (j & 3))) & 255u);
                 } else if constexpr (!R::KQ) {
                     if (R::F32 ? !ONE || j + WK == 8 : (j + 1) % SEG == 0) s = h2f(EARLY ? sv[r] : lds<uint16_t>(cur, pS + e * 32));
-                    if (ONE && j + WK == 8) rs[r] = s;
+                    if (SEG0 == 8 && j + WK == 8) rs[r] = s;
                 }
                 if constexpr (R::A16) {
                     // sum 256 hi w and sum lo w over the group's chunks (256 inputs at most), each exact
@@ -633,12 +643,12 @@ __global__ __launch_bounds__(WT * WR * WK * 64, Tr<F>::F32 ? 4 : 2) void gemm_pl
                     v4f xh[TT], xl[TT];
 #pragma unroll
                     for (int t = 0; t < TT; t++)
-                        xh[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, ap[t][0]), b,
+                        xh[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, ah[t]), b,
                                                                        j % SEG == 0 ? zero : seg[t][r], 0, 0, 0);
 #pragma unroll
                     for (int t = 0; t < TT; t++)
                         xl[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
-                            __builtin_bit_cast(v8h, ap[t][1]), b, one ? xh[t] : j % SEG == 0 ? zero : sel[t][r], 0, 0, 0);
+                            __builtin_bit_cast(v8h, al[t]), b, one ? xh[t] : j % SEG == 0 ? zero : sel[t][r], 0, 0, 0);
 #pragma unroll
                     for (int t = 0; t < TT; t++) {
                         if ((j + 1) % SEG == 0) {  // tile_i16's flush
@@ -677,10 +687,11 @@ __global__ __launch_bounds__(WT * WR * WK * 64, Tr<F>::F32 ? 4 : 2) void gemm_pl
                     }
                 } else {
 #pragma unroll
-                    for (int q = 0; q < 2; q++)
+                    for (int t = 0; t < TT; t++)
+                        x[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, ah[t]), b, x[t], 0, 0, 0);
 #pragma unroll
-                        for (int t = 0; t < TT; t++)
-                            x[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, ap[t][q]), b, x[t], 0, 0, 0);
+                    for (int t = 0; t < TT; t++)
+                        x[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, al[t]), b, x[t], 0, 0, 0);
                 }
                 if constexpr (CHAIN) {
 #pragma unroll

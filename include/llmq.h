@@ -179,16 +179,15 @@ LLMQ_API int llmq_linear(llmq_ctx *ctx, float *out, const float *x, const llmq_m
  * harnesses that forbid hipMalloc).  Same arguments, kernels and results
  * (bit for bit) as llmq_linear; where llmq_linear grows the context's
  * workspace (the a16 prompt GEMM's int16 activation codes, row scales and
- * fp16 planes, the Q4_K matmul's fp16 activation record), this form uses a fixed
- * per-GPU scratch array of LLMQ_NOALLOC_SCRATCH_BYTES that each GPU the
+ * fp16 planes, the Q4_K matmul's fp16 activation record), this form uses a
+ * fixed per-GPU scratch array of LLMQ_NOALLOC_SCRATCH_BYTES that each GPU the
  * library runs on holds until the process ends.  It calls no hipMalloc /
  * hipFree.  Sizes needing more scratch than that (a16: T x IN x 2 bytes
  * and T x 4, each rounded up to 256; Q4_K: the record's ~4.4 x T x IN
  * bytes, T rounded up to 16) return LLMQ_EINVAL; the other formats use no
- * scratch.  An a16 matrix
- * in groups of 32, or of whole 256-input superblocks, also puts its prompt
- * GEMM's fp16 activation planes there (T x IN x 4 bytes, T rounded up to 16)
- * when they fit, else runs the int8-MFMA form of the GEMM (the same bits).
+ * scratch.  An a16 matrix in groups of 32, or of whole 256-input superblocks,
+ * also puts its prompt GEMM's fp16 activation planes there (T x IN x 4 bytes,
+ * T rounded up to 16) when they fit, else runs the int8-MFMA form of the GEMM (the same bits).
  * Every call that uses it shares the array: calls that overlap in time on one
  * GPU (different streams or threads) race; calls ordered on one stream do
  * not.  Nothing in the scratch needs to start at zero (each call writes all
